@@ -39,7 +39,7 @@ def listed():
         # the 2D circle that the reference runs on the CPU, with the force logged at every step
         _case("circle_192x128_forces", n=(192, 128), steps=8, forces=True),
         # a 2D double-precision validation run with a convective exit, on a ragged grid
-        _case("ellipse_328x136_f64_exit", n=(328, 136), dtype="f64", steps=6, exit_bc=True, body="ellipsoid"),
+        _case("ellipse_352x144_f64_exit", n=(352, 144), dtype="f64", steps=6, exit_bc=True, body="ellipsoid"),
         # a large 2D wake, the body measured again at every step (sim_step's default)
         _case("circle_1024x512_remeasure", n=(1024, 512), steps=6, remeasure=True),
         # a small 3D sphere, the size of the introductory example
@@ -62,9 +62,13 @@ def listed():
     ]
 
 
-def _spread(rng, lo, hi, step):
-    """A multiple of `step` in [lo, hi], spread over the logarithm."""
-    return max(lo, step * round(math.exp(rng.uniform(math.log(lo), math.log(hi))) / step))
+SIZES = sorted({a << k for a in (1, 3, 5, 7, 9, 11, 13, 15) for k in range(3, 11)})  # a·2ⁿ, as multigrid asks for
+
+
+def _spread(rng, lo, hi):
+    """A size in [lo, hi], spread over the logarithm."""
+    at = rng.uniform(math.log(lo), math.log(hi))
+    return min((v for v in SIZES if lo <= v <= hi), key=lambda v: abs(math.log(v) - at))
 
 
 def draw(rng):
@@ -74,17 +78,16 @@ def draw(rng):
     if kind == "batch":
         return _case(kind="batch", n=(512, 256), steps=rng.randint(4, 16), members=rng.randint(3, 64))
     if kind == "2d":
-        nx = _spread(rng, 64, 1536, 8)
-        n = (nx, _spread(rng, max(48, nx // 3), max(64, nx), 8))
+        nx = _spread(rng, 64, 1536)
+        n = (nx, _spread(rng, max(48, nx // 3), max(64, nx)))
         return _case(n=n, dtype=dtype, scheme=scheme, steps=rng.randint(3, 8), remeasure=rng.random() < 0.4,
                      exit_bc=rng.random() < 0.3, forces=rng.random() < 0.3, mean=rng.random() < 0.2,
                      body=rng.choice(["sphere", "ellipsoid"]))
     if kind == "vortices":
-        m = _spread(rng, 32, 192, 8)
-        n = (m, _spread(rng, 32, 192, 16)) + ((_spread(rng, 32, 160, 16),) if rng.random() < 0.7 else ())
+        n = (_spread(rng, 32, 192), _spread(rng, 32, 192)) + ((_spread(rng, 32, 160),) if rng.random() < 0.7 else ())
         return _case(kind="vortices", n=n, dtype=dtype, scheme=scheme, steps=rng.randint(2, 5))
-    nx = _spread(rng, 64, 384, 8)
-    n = (nx, _spread(rng, 48, max(56, nx * 2 // 3), 8), _spread(rng, 32, max(48, nx // 2), 8))
+    nx = _spread(rng, 64, 384)
+    n = (nx, _spread(rng, 48, max(56, nx * 2 // 3)), _spread(rng, 32, max(48, nx // 2)))
     mixed = dtype == "f32" and rng.random() < 0.25
     return _case(n=n, dtype=dtype, scheme=scheme, steps=rng.randint(2, 5), remeasure=rng.random() < 0.3,
                  exit_bc=not mixed and rng.random() < 0.3, solver="mixed" if mixed else "plain",
