@@ -199,20 +199,24 @@ __global__ void __launch_bounds__(256) kb_prolong(const ALev<T>* __restrict__ A,
   else
     k_prolong_inc_body<T, false>(a.g, a.gc, a.t, a.cm, a.perdir, a.L, a.r, a.x, a.e, a.xc, a.wp, b.lid);
 }
-// the coarse tail of each simulation: one workgroup per simulation (k_mg_tail_lds)
+// the coarse tail of each simulation: one workgroup per simulation (k_mg_tail_fast, or k_mg_tail_lds
+// where its first level has more x pairs than threads)
 template <class T>
 struct ATail {
   TailDesc<T> d;
+  TailFast<T> f;
   const T* wp;
-  int bx, by, bz;
+  int fast;
 };
-template <class T>
+template <class T, int D>
 __global__ void __launch_bounds__(1024) kb_mg_tail(const ATail<T>* __restrict__ A, const int* __restrict__ sims,
                                                    const int* __restrict__ act) {
   const int s = sims[blockIdx.x];
   if (act && !act[s]) return;
   const ATail<T>& a = A[blockIdx.x];
-  k_mg_tail_lds_body<T>(a.d, a.wp, a.bx, a.by, a.bz);
+  __shared__ double cg[5][TAIL_CG_MAX];
+  if (a.fast) k_mg_tail_fast_body<T, D>(a.f, a.wp, cg);
+  else k_mg_tail_lds_body<T, D, false>(a.d, a.wp, cg);
 }
 
 template <class T>

@@ -257,19 +257,54 @@ struct MG {
     dfree(x64[1]);
     dfree(c_alt);
     dfree(r_alt);
-    for (auto& l : lv) {
+    dfree(arena);
+    dfree(tail_img);
+    dfree(row_arena);
+    for (size_t k = 0; k < lv.size(); ++k) {
+      Level<T>& l = lv[k];
+      dfree(l.e2);
+      dfree(l.ej);
+      if (k > 0) continue;  // the coarse levels' arrays lie in the arenas
       if (l.ownL) dfree(l.L);
       if (l.ownx) dfree(l.x);
       if (l.ownz) dfree(l.z);
       dfree(l.r);
       dfree(l.e);
-      dfree(l.e2);
-      dfree(l.ej);
       dfree(l.lrow);
     }
   }
 
   static bool divisible(int N) { return N % 2 == 0 && N > 4; }  // src/MultiLevelPoisson.jl:52
+
+  // The coarse levels' arrays in one allocation, and their row flags in another: the passes over
+  // small levels are bound by latency, and the coarse tail reads the arrays of all its levels at its
+  // start, so they share as few memory pages as they can.
+  T* arena = nullptr;
+  uint8_t* row_arena = nullptr;
+  void place_coarse(int D) {
+    auto pad = [](int64_t v) { return (v + 63) & ~(int64_t)63; };
+    for (int pass = 0; pass < 2; ++pass) {  // sizes, then addresses; the coarsest levels first
+      int64_t o = 0, ro = 0;
+      for (size_t k = lv.size() - 1; k >= 1; --k) {
+        Level<T>& l = lv[k];
+        const int64_t n = pad(l.g.n), nL = pad(l.g.n * D), nr = pad(2 * (int64_t)l.g.N[1] * l.g.N[2]);
+        if (pass == 1) {
+          l.L = arena + o;
+          l.r = l.L + nL;
+          l.x = l.r + n;
+          l.e = l.x + n;
+          l.z = l.e + n;
+          l.lrow = row_arena + ro;
+        }
+        o += nL + 4 * n;
+        ro += nr;
+      }
+      if (pass == 0) {
+        arena = dalloc<T>(o);
+        row_arena = dalloc<uint8_t>(ro);
+      }
+    }
+  }
 
   // Level sizes (src/MultiLevelPoisson.jl:33-41,61-77); level 0 arrays may be supplied.
   void build(int D, const int* Ng, T* L0, T* x0, T* z0, int maxlevels = 10) {
@@ -320,12 +355,6 @@ struct MG {
       lv.back().cmask = cm;
       Level<T> lc;
       lc.g = make_geo(D, Na);
-      lc.L = dalloc<T>(lc.g.n * D);
-      lc.x = dalloc<T>(lc.g.n);
-      lc.z = dalloc<T>(lc.g.n);
-      lc.r = dalloc<T>(lc.g.n);
-      lc.e = dalloc<T>(lc.g.n);
-      lc.lrow = dalloc<uint8_t>(2 * (int64_t)lc.g.N[1] * lc.g.N[2]);
       // restrictL of a uniform fine level: Σ over the 2 children of each coarsened transverse
       // direction, halved when the face's own direction is coarsened (all powers of two: exact)
       const Level<T>& fl = lv.back();
@@ -338,6 +367,7 @@ struct MG {
       lv.push_back(lc);
     }
     if (lv.size() <= 2) throw WlErr(WL_EINVAL, "MultiLevelPoisson requires size=a2ⁿ, where n>2");
+    place_coarse(D);
     for (size_t l = 0; l < lv.size(); ++l)  // before any graph capture: no allocation while capturing
       if (gs_pair_ok((int)l) || gs_dbl_ok((int)l)) lv[l].e2 = dalloc<T>(lv[l].g.n);
     if (fold_coarse_inc && pairs_ok(0)) lv[0].ej = dalloc<T>(lv[0].g.n);
@@ -358,8 +388,10 @@ struct MG {
     }
     static bool attr_set = false;  // the LDS tail may use more than 64 KB of dynamic LDS
     if (!attr_set) {
-      HIPCK(hipFuncSetAttribute((const void*)k_mg_tail_lds<T>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                TAIL_LDS_BYTES));
+      for (const void* k : {(const void*)k_mg_tail_lds<T, 2, false>, (const void*)k_mg_tail_lds<T, 2, true>,
+                            (const void*)k_mg_tail_lds<T, 3, false>, (const void*)k_mg_tail_lds<T, 3, true>,
+                            (const void*)k_mg_tail_fast<T, 2>, (const void*)k_mg_tail_fast<T, 3>})
+        HIPCK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, TAIL_LDS_BYTES));
       attr_set = true;
     }
   }
@@ -478,6 +510,7 @@ struct MG {
       bc_vec(c.g, c.L, zero, 0);
     }
     for (size_t l = 0; l < lv.size(); ++l) build_lrows((int)l);
+    build_tail_image();
   }
 
   // mode 0: Σ into dsc[slot]; 1: also the mean and its flag (tsc[0..1]); 2 and 3 (slot 1): then the
@@ -692,11 +725,29 @@ struct MG {
   // First level run by the single-workgroup coarse tail: the first level (>= 1) from which every
   // coarser level fits the tail's LDS image; WL_TAIL_CELLS (cells of the first tail level) makes
   // it a global-memory tail from that size instead.  -1: no tail.
+  // A flow's solver starts it, where such a level exists, at the first one that also has at most
+  // one x pair per thread (k_mg_tail_fast).
   int64_t tail_cells = -1;  // WL_TAIL_CELLS when the solver was built (-1: unset)
+  static int log2_up_h(int v) {
+    int k = 0;
+    while ((1 << k) < v) ++k;
+    return k;
+  }
+  static int tail_threads(const Geo& g) {  // threads a level takes with one x pair each
+    const int lx = log2_up_h((g.N[0] - 1) / 2), ly = log2_up_h(g.N[1] - 2);
+    const int64_t t = ((int64_t)(g.D == 3 ? g.N[2] - 2 : 1)) << (lx + ly);
+    return (int)std::min<int64_t>(t, 1 << 20);
+  }
+  bool tail_fast(int l) const {
+    return fold_coarse_inc && tail_threads(lv[l].g) <= TAIL_FAST_PAIRS && tail_bytes(l) <= TAIL_LDS_BYTES;
+  }
   int tail_start(bool* in_lds) const {
     const int64_t cells = tail_cells;
     *in_lds = false;
     if (cells == 0) return -1;
+    if (cells < 0)
+      for (size_t l = 1; l < lv.size(); ++l)
+        if (tail_fast((int)l)) { *in_lds = true; return (int)l; }
     if (cells > 0) {
       for (size_t l = 1; l < lv.size(); ++l)
         if (lv[l].g.n <= cells) return (int)l;
@@ -706,9 +757,71 @@ struct MG {
       if (tail_bytes((int)l) <= TAIL_LDS_BYTES) { *in_lds = true; return (int)l; }
     return -1;
   }
+  // the fast tail's image of L, D and 1/D (k_tail_image), formed with L in update()
+  T* tail_img = nullptr;
+  TailFast<T> tail_desc(int Lt) const {
+    TailFast<T> d;
+    std::memset(&d, 0, sizeof(d));
+    d.n = (int)lv.size() - Lt;
+    d.perdir = perdir;
+    int o = 0;
+    for (int k = 0; k < d.n; ++k) {
+      const Geo& g = lv[Lt + k].g;
+      TailLv& q = d.lv[k];
+      q.N0 = g.N[0]; q.N1 = g.N[1]; q.N2 = g.N[2];
+      q.s1 = (int)g.s[1]; q.s2 = (int)g.s[2]; q.n = (int)g.n; q.cm = lv[Lt + k].cmask;
+      q.lx = log2_up_h((g.N[0] - 1) / 2); q.ly = log2_up_h(g.N[1] - 2);
+      q.small = tail_threads(g) <= TAIL_WAVE_PAIRS;
+      q.oL = o;
+      q.oD = o + g.D * q.n;
+      q.oI = q.oD + q.n;
+      o = q.oI + q.n;
+    }
+    o = (o + 3) & ~3;
+    d.nimg = o;
+    for (int k = 0; k < d.n; ++k) {
+      TailLv& q = d.lv[k];
+      q.oR = o;
+      q.oX = o + q.n;
+      q.oE = q.oX + q.n;
+      o = q.oE + q.n;
+    }
+    d.img = tail_img;
+    d.r = lv[Lt].r;
+    d.x = lv[Lt].x;
+    return d;
+  }
+  static size_t tail_desc_lds(const TailFast<T>& d) {
+    const TailLv& q = d.lv[d.n - 1];
+    return (size_t)(q.oE + q.n) * sizeof(T);
+  }
+  void build_tail_image() {
+    bool in_lds = false;
+    const int Lt = tail_start(&in_lds);
+    if (Lt < 1 || !in_lds || !tail_fast(Lt)) return;
+    TailFast<T> d = tail_desc(Lt);
+    if (!tail_img) tail_img = dalloc<T>(d.nimg);
+    for (int k = 0; k < d.n; ++k) {
+      const Level<T>& q = lv[Lt + k];
+      hipLaunchKernelGGL(k_tail_image<T>, dim3((unsigned)((q.g.n + 255) / 256)), dim3(256), 0, st, q.g,
+                         (const T*)q.L, tail_img + d.lv[k].oL);
+      KCK();
+    }
+  }
   bool exact_coarsest = false;  // set by the mixed-precision loop around its V-cycles
   bool coarse_pcg = false;      // WL_COARSE_PCG=1: that coarsest level by FP64 pcg! instead of GS-RB
   void launch_tail(int Lt, bool in_lds, const T* w) {
+    if (in_lds && tail_fast(Lt)) {
+      TailFast<T> f = tail_desc(Lt);
+      f.exact = exact_coarsest ? (coarse_pcg ? 2 : 1) : 0;
+      ProfScope ps(P, st, "mg_tail", Lt, 0.0);
+      if (lv[Lt].g.D == 3)
+        hipLaunchKernelGGL((k_mg_tail_fast<T, 3>), dim3(1), dim3(TAIL_FAST_PAIRS), tail_desc_lds(f), st, f, w);
+      else
+        hipLaunchKernelGGL((k_mg_tail_fast<T, 2>), dim3(1), dim3(TAIL_FAST_PAIRS), tail_desc_lds(f), st, f, w);
+      KCK();
+      return;
+    }
     TailDesc<T> d;
     d.n = (int)lv.size() - Lt;
     d.perdir = perdir;
@@ -727,8 +840,15 @@ struct MG {
     }
     ProfScope ps(P, st, "mg_tail", Lt, 0.0);
     if (in_lds) {
-      const int bx = lv[Lt].g.D == 3 ? 16 : 32, by = lv[Lt].g.D == 3 ? 8 : 32, bz = lv[Lt].g.D == 3 ? 8 : 1;
-      hipLaunchKernelGGL(k_mg_tail_lds<T>, dim3(1), dim3(1024), (size_t)(off * sizeof(T)), st, d, w, bx, by, bz);
+      // a standalone MultiLevelPoisson keeps its coarse levels' whole state
+      const size_t lds = (size_t)(off * sizeof(T));
+      if (lv[Lt].g.D == 3) {
+        if (fold_coarse_inc) hipLaunchKernelGGL((k_mg_tail_lds<T, 3, false>), dim3(1), dim3(1024), lds, st, d, w);
+        else hipLaunchKernelGGL((k_mg_tail_lds<T, 3, true>), dim3(1), dim3(1024), lds, st, d, w);
+      } else {
+        if (fold_coarse_inc) hipLaunchKernelGGL((k_mg_tail_lds<T, 2, false>), dim3(1), dim3(1024), lds, st, d, w);
+        else hipLaunchKernelGGL((k_mg_tail_lds<T, 2, true>), dim3(1), dim3(1024), lds, st, d, w);
+      }
     } else
       hipLaunchKernelGGL((k_mg_tail<T, false>), dim3(1), dim3(1024), 0, st, d, w);
     KCK();
@@ -2150,8 +2270,8 @@ struct BatchT : BatchBase {
         }
         tail_lds = std::max(tail_lds, (size_t)(off * sizeof(T)));
         t.wp = (const T*)F[s]->B.tsc + 3;
-        const bool d3 = mg.lv[Lt[s]].g.D == 3;
-        t.bx = d3 ? 16 : 32; t.by = d3 ? 8 : 32; t.bz = d3 ? 8 : 1;
+        t.fast = mg.tail_fast(Lt[s]) ? 1 : 0;
+        if (t.fast) t.f = mg.tail_desc(Lt[s]);
         a.push_back(t);
         sims.push_back(s);
       }
@@ -2159,7 +2279,8 @@ struct BatchT : BatchBase {
       tail_sims = upload(sims);
       static bool attr = false;
       if (!attr) {
-        HIPCK(hipFuncSetAttribute((const void*)kb_mg_tail<T>, hipFuncAttributeMaxDynamicSharedMemorySize, TAIL_LDS_BYTES));
+        for (const void* k : {(const void*)kb_mg_tail<T, 2>, (const void*)kb_mg_tail<T, 3>})
+          HIPCK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, TAIL_LDS_BYTES));
         attr = true;
       }
     }
@@ -2350,7 +2471,10 @@ struct BatchT : BatchBase {
         KCK();
       }
     }
-    hipLaunchKernelGGL(kb_mg_tail<T>, dim3(ns), dim3(1024), tail_lds, st, tails, tail_sims, (const int*)act);
+    if (D == 3)
+      hipLaunchKernelGGL((kb_mg_tail<T, 3>), dim3(ns), dim3(1024), tail_lds, st, tails, tail_sims, (const int*)act);
+    else
+      hipLaunchKernelGGL((kb_mg_tail<T, 2>), dim3(ns), dim3(1024), tail_lds, st, tails, tail_sims, (const int*)act);
     KCK();
     for (int c = Cmax; c >= 1; --c) {  // members with c < Lt: smooth!(c); members with c <= Lt: prolongate!
       if (gs[c].nblk) gs_sweeps(c);  // their last increment! is folded into the prolongation below
