@@ -1,5 +1,6 @@
 """The coarse levels of a flow's V-cycle on the GPU: the single-workgroup tail (k_mg_tail_fast and
-its general form), bit for bit against the oracle at the sizes where its thread maps end."""
+its general form) and the fused up-leg of a level (k_up), bit for bit against the oracle at the
+sizes where their tiles and thread maps end."""
 import os
 
 import numpy as np
@@ -21,7 +22,7 @@ def wl():
 CASES = [
     # the smallest hierarchy: the tail is level 1 on
     ((8, 8), {}), ((8, 8, 8), {}),
-    # ragged coarsening
+    # around one and two tiles of k_up (54 x 22 and 24 x 8 x 8 cells), ragged coarsening
     ((52, 20), {}), ((56, 24), {}), ((108, 44), {}), ((24, 8, 8), {}), ((26, 10, 12), {}),
     # odd extents: directions that never coarsen, half_rangek short of the last plane
     ((64, 33), {}), ((33, 64), {}), ((32, 16, 17), {}), ((17, 32, 16), {}),

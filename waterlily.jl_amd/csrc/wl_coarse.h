@@ -1,5 +1,5 @@
 // The coarse end of the V-cycle, where a pass over a level costs its latency and not its bytes:
-// the single-workgroup tail (k_mg_tail_fast, and its general form k_mg_tail_lds).
+// the single-workgroup tail (k_mg_tail_lds) and the fused up-leg of a level (k_up).
 //
 // Included by wl_kernels.h after the per-cell pieces it uses (LRows, lcell, pro_map, TailDesc).
 #pragma once
@@ -763,6 +763,244 @@ template <class T, int D>
 __global__ void __launch_bounds__(TAIL_FAST_PAIRS) k_mg_tail_fast(TailFast<T> d, const T* __restrict__ wp) {
   __shared__ double cg[5][TAIL_CG_MAX];
   k_mg_tail_fast_body<T, D>(d, wp, cg);
+}
+
+// ---- the up-leg of one level in one launch ----
+// prolongate! from level l+1, increment!(l), ϵ = r·iD, the four GS-RB half sweeps and smooth!'s
+// increment! of a flow's own solver (src/MultiLevelPoisson.jl:98-100, src/Poisson.jl:100-148); x of
+// the level comes out final, r and ϵ stay on the chip (the next V-cycle overwrites them).
+//
+// As separate launches (one prolongation, four half sweeps, the increment in the next finer
+// prolongation) a level below a million cells costs five launches of 3-5 us, each moving a few MB
+// that sit in the caches.  Here a block takes a region of 64 x 32 cells (2D) or 16 x 16 x 12 (3D)
+// around its output tile: stage s of a cell needs stage s − 1 of its neighbours, so the halo is the
+// four half sweeps' (FIN: one more, for the residual), which the blocks recompute.  A thread owns
+// x pairs of the region (one in 2D, two in 3D), one cell of which each half sweep updates, and
+// keeps their residuals, 1/D and coefficients in registers; the LDS carries ϵ, and before it the
+// prolonged coarse values.  Every value is formed by the operations of the separate passes in their
+// order, so the results are the same bits.
+//
+// FIN (the finest level): also r −= ω·Aϵ into rout (the neighbouring blocks still read r), the next
+// Jacobi!'s ϵ = r·iD into ej and the block's Σr² into partial.
+// Periodic directions: ghosts hold perBC!'s image of the first ϵ for all four half sweeps, as in the
+// reference; FIN needs the images of the last and takes no periodic directions.
+template <class T>
+struct UpArgs {
+  Geo gf, gc;
+  int cm, perdir;
+  LRows<T> L;
+  const T* r;
+  T* x;
+  const T* xc;
+  const T* w;
+  T* rout;
+  T* ej;
+  double* partial;
+  int ntx, nty;  // output tiles in x and y
+};
+template <int D, bool FIN>
+struct UpTile {
+  static constexpr int H = FIN ? 5 : 4;
+  static constexpr int LX = D == 3 ? 3 : 5, LY = D == 3 ? 4 : 5;  // log2 of the pairs and rows
+  static constexpr int RX = 2 << LX, RY = 1 << LY, RZ = D == 3 ? 12 : 1;
+  static constexpr int OX = RX - 2 * H, OY = RY - 2 * H, OZ = D == 3 ? RZ - 2 * H : 1;
+  static constexpr int SX = RX + 2, SY = RY + 2, SZ = D == 3 ? RZ + 2 : 1;  // with a ring of one cell
+  static constexpr int NI = D == 3 ? 2 : 1, DZ = RZ / NI;                   // pairs per thread, planes apart
+  static constexpr int THREADS = (RX / 2) * RY * DZ;
+};
+template <class T, int D, bool FIN>
+constexpr size_t up_lds() {
+  using U = UpTile<D, FIN>;
+  return sizeof(T) * U::SX * U::SY * U::SZ;
+}
+// The face coefficients of an x pair (cells 0 and 1): x faces x0, x1, x2; y and z faces low and high
+template <class T, int D>
+struct PairCoef {
+  T x0, x1, x2, yl[2], yh[2], zl[D == 3 ? 2 : 1], zh[D == 3 ? 2 : 1];
+  __device__ __forceinline__ T diag(int c) const {
+    T s = 0;
+    s -= ((c ? x1 : x0) + (c ? x2 : x1));
+    s -= (yl[c] + yh[c]);
+    if constexpr (D == 3) s -= (zl[c] + zh[c]);
+    return s;
+  }
+  // x(I)·D + Σ_i (x(I−e_i)·L[I,i] + x(I+e_i)·L[I+e_i,i]) at cell c, where p stands (s = x(I)·D)
+  __device__ __forceinline__ T mult(int c, T s, const T* p, int sy, int sz) const {
+    s += (p[-1] * (c ? x1 : x0) + p[1] * (c ? x2 : x1));
+    s += (p[-sy] * yl[c] + p[sy] * yh[c]);
+    if constexpr (D == 3) s += (p[-sz] * zl[c] + p[sz] * zh[c]);
+    return s;
+  }
+  // gauss (src/Poisson.jl:116-122) before the product with iD; first: cell 0, where p stands
+  __device__ __forceinline__ T gauss(bool first, T s, const T* p, int sy, int sz) const {
+    const T xm = p[-1], xp = p[1], ym = p[-sy], yp = p[sy];
+    T zm = T(0), zp = T(0);
+    if constexpr (D == 3) {
+      zm = p[-sz];
+      zp = p[sz];
+    }
+    s -= (xm * (first ? x0 : x1) + xp * (first ? x1 : x2));
+    s -= (ym * (first ? yl[0] : yl[1]) + yp * (first ? yh[0] : yh[1]));
+    if constexpr (D == 3) s -= (zm * (first ? zl[0] : zl[1]) + zp * (first ? zh[0] : zh[1]));
+    return s;
+  }
+};
+// from the two cells' own coefficients; h of cell 0 and l of cell 1 in x are one face, taken from
+// cell 0 where it has a value (va)
+template <class T, int D>
+__device__ __forceinline__ PairCoef<T, D> pair_coef(const LC<T>& a, const LC<T>& b, bool va) {
+  PairCoef<T, D> c;
+  c.x0 = a.l[0]; c.x1 = va ? a.h[0] : b.l[0]; c.x2 = b.h[0];
+  c.yl[0] = a.l[1]; c.yh[0] = a.h[1]; c.yl[1] = b.l[1]; c.yh[1] = b.h[1];
+  if constexpr (D == 3) {
+    c.zl[0] = a.l[2]; c.zh[0] = a.h[2]; c.zl[1] = b.l[2]; c.zh[1] = b.h[2];
+  }
+  return c;
+}
+template <class T, int D, bool FIN>
+__device__ __forceinline__ void k_up_body(const UpArgs<T>& a, int bid, int nb, int pidx) {
+  using U = UpTile<D, FIN>;
+  constexpr int H = U::H, NI = U::NI, SX = U::SX, SXY = U::SX * U::SY;
+  extern __shared__ __align__(16) unsigned char up_smem[];
+  T* const S = reinterpret_cast<T*>(up_smem);  // SXY·SZ values
+  const T w = *a.w;
+  const int tid = threadIdx.x;
+  const int N[3] = {a.gf.N[0], a.gf.N[1], a.gf.N[2]};
+  const int lid = xcd_tile_of(bid, nb);
+  const int tx = lid % a.ntx, t1 = lid / a.ntx, ty = t1 % a.nty, tz = t1 / a.nty;
+  // the region's first cell
+  const int bx = 1 + tx * U::OX - H, by = 1 + ty * U::OY - H, bz = D == 3 ? 1 + tz * U::OZ - H : 0;
+  // the inside cell whose value stands at coordinate c of direction q: itself, the image of a
+  // periodic ghost (or of the cell one beyond it), or none (−1)
+  auto image = [&](int c, int q) -> int {
+    const int n = N[q];
+    if (c >= 1 && c <= n - 2) return c;
+    if (!((a.perdir >> q) & 1) || c < -1 || c > n) return -1;
+    return c < 1 ? c + (n - 2) : c - (n - 2);
+  };
+  // ---- the prolonged coarse values of the region and one cell around it ----
+  {
+    constexpr int NS = SXY * U::SZ;
+#pragma unroll 4
+    for (int k = tid; k < NS; k += U::THREADS) {
+      const int cx = image(bx - 1 + k % SX, 0), cy = image(by - 1 + (k / SX) % U::SY, 1);
+      const int cz = D == 3 ? image(bz - 1 + k / SXY, 2) : 0;
+      const bool ok = cx >= 0 && cy >= 0 && cz >= 0;
+      const int qx = (a.cm & 1) ? (cx + 1) >> 1 : cx, qy = (a.cm & 2) ? (cy + 1) >> 1 : cy;
+      const int qz = D == 3 ? ((a.cm & 4) ? (cz + 1) >> 1 : cz) : 0;
+      const T v = a.xc[ok ? qx + a.gc.s[1] * qy + a.gc.s[2] * qz : 0];
+      S[k] = ok ? v : T(0);
+    }
+  }
+  const int lp = tid & ((1 << U::LX) - 1), ly = (tid >> U::LX) & ((1 << U::LY) - 1), lz0 = D == 3 ? tid >> (U::LX + U::LY) : 0;
+  const int cx = bx + 2 * lp, cy = by + ly;
+  const int s0 = 1 + 2 * lp + SX * (1 + ly);  // LDS index of the pair's first cell in plane −1 (3D) or 0
+  const int mxa = image(cx, 0), mxb = image(cx + 1, 0), my = image(cy, 1);
+  const int klim = D == 3 ? 2 * (N[2] / 2) - 2 : 2 * (N[1] / 2) - 2;
+  const bool ixa = cx >= 1 && cx <= N[0] - 2, ixb = cx + 1 >= 1 && cx + 1 <= N[0] - 2, iy = cy >= 1 && cy <= N[1] - 2;
+  T ra[NI], rb[NI], ia[NI], ib[NI], xa[NI], xb[NI];
+  PairCoef<T, D> C[NI];
+  // a cell without a value takes the first inside cell's coefficients; its ϵ is set to 0 below
+  auto coef = [&](int i) -> PairCoef<T, D> {
+    const int mz = D == 3 ? image(bz + lz0 + U::DZ * i, 2) : 0;
+    const bool row = my >= 0 && mz >= 0;
+    const int y = row ? my : 1, z = D == 3 ? (row ? mz : 1) : 0;
+    return pair_coef<T, D>(lcell(a.gf, a.L, row && mxa >= 0 ? mxa : 1, y, z),
+                           lcell(a.gf, a.L, row && mxb >= 0 ? mxb : 1, y, z), mxa >= 0);
+  };
+  uint32_t fl = 0;  // per pair: 1, 2 updated by the sweeps; 4, 8 output cells
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {  // the pairs' own loads, before the barrier
+    const int cz = D == 3 ? bz + lz0 + U::DZ * i : 0;
+    const int mz = D == 3 ? image(cz, 2) : 0;
+    const bool iz = D == 2 || (cz >= 1 && cz <= N[2] - 2);
+    const bool row = my >= 0 && mz >= 0;
+    const bool reach = (D == 3 ? cz : cy) <= klim;
+    const bool oy = ly >= H && ly < H + U::OY && (D == 2 || (lz0 + U::DZ * i >= H && lz0 + U::DZ * i < H + U::OZ));
+    const bool in = iy && iz;
+    const bool oa = in && ixa && oy && 2 * lp >= H && 2 * lp < H + U::OX;
+    const bool ob = in && ixb && oy && 2 * lp + 1 >= H && 2 * lp + 1 < H + U::OX;
+    fl |= (uint32_t)((in && ixa && reach ? 1 : 0) | (in && ixb && reach ? 2 : 0) | (oa ? 4 : 0) | (ob ? 8 : 0)) << (4 * i);
+    const int64_t rowI = row ? a.gf.s[1] * my + a.gf.s[2] * mz : 0;
+    const bool va = row && mxa >= 0, vb = row && mxb >= 0;
+    ra[i] = va ? a.r[rowI + mxa] : T(0);
+    rb[i] = vb ? a.r[rowI + mxb] : T(0);
+    xa[i] = oa ? a.x[rowI + mxa] : T(0);
+    xb[i] = ob ? a.x[rowI + mxb] : T(0);
+    C[i] = coef(i);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {  // increment! with the prolonged values, ϵ = r·iD
+    const T* p = S + s0 + (D == 3 ? SXY * (1 + lz0 + U::DZ * i) : 0);
+    const PairCoef<T, D>& c = C[i];
+    const T e0 = p[0], e1 = p[1];
+    const T Da = c.diag(0), Db = c.diag(1);
+    ra[i] = ra[i] - w * c.mult(0, e0 * Da, p, SX, SXY);
+    rb[i] = rb[i] - w * c.mult(1, e1 * Db, p + 1, SX, SXY);
+    xa[i] = xa[i] + w * e0;
+    xb[i] = xb[i] + w * e1;
+    ia[i] = inv_diag(Da);
+    ib[i] = inv_diag(Db);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {  // ghosts and cells beyond hold 0; periodic ghosts their image's ϵ
+    const int cz = D == 3 ? bz + lz0 + U::DZ * i : 0;
+    const bool row = my >= 0 && (D == 2 || image(cz, 2) >= 0);
+    T* p = S + s0 + (D == 3 ? SXY * (1 + lz0 + U::DZ * i) : 0);
+    p[0] = row && mxa >= 0 ? ra[i] * ia[i] : T(0);
+    p[1] = row && mxb >= 0 ? rb[i] * ib[i] : T(0);
+  }
+  __syncthreads();
+#pragma unroll 1
+  for (int it = 1; it <= 4; ++it) {
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int cz = D == 3 ? bz + lz0 + U::DZ * i : 0;
+      const bool fa = ((cx + cy + cz + it + D + 1) & 1) == 0;  // the pair's cell of this sweep's colour
+      if ((fl >> (4 * i + (fa ? 0 : 1))) & 1) {
+        T* p = S + s0 + (D == 3 ? SXY * (1 + lz0 + U::DZ * i) : 0) + (fa ? 0 : 1);
+        const T s = C[i].gauss(fa, fa ? ra[i] : rb[i], p, SX, SXY);
+        p[0] = s * (fa ? ia[i] : ib[i]);
+      }
+    }
+    if (it < 4 || FIN) __syncthreads();
+  }
+  double acc = 0;
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {  // smooth!'s increment!
+    const int cz = D == 3 ? bz + lz0 + U::DZ * i : 0;
+    const bool oa = (fl >> (4 * i)) & 4, ob = (fl >> (4 * i)) & 8;
+    const T* p = S + s0 + (D == 3 ? SXY * (1 + lz0 + U::DZ * i) : 0);
+    const int64_t I = cx + a.gf.s[1] * cy + a.gf.s[2] * cz;
+    const T e0 = p[0], e1 = p[1];
+    if (oa) a.x[I] = xa[i] + w * e0;
+    if (ob) a.x[I + 1] = xb[i] + w * e1;
+    if (FIN) {
+      const PairCoef<T, D>& c = C[i];
+      const T na = ra[i] - w * c.mult(0, e0 * c.diag(0), p, SX, SXY);
+      const T nb2 = rb[i] - w * c.mult(1, e1 * c.diag(1), p + 1, SX, SXY);
+      if (oa) {
+        a.rout[I] = na;
+        a.ej[I] = na * ia[i];
+        acc += (double)na * (double)na;
+      }
+      if (ob) {
+        a.rout[I + 1] = nb2;
+        a.ej[I + 1] = nb2 * ib[i];
+        acc += (double)nb2 * (double)nb2;
+      }
+    }
+  }
+  if (FIN) {
+    const double t = block_sum(acc);
+    if (tid == 0) a.partial[pidx] = t;
+  }
+}
+template <class T, int D, bool FIN>
+__global__ void __launch_bounds__((UpTile<D, FIN>::THREADS)) k_up(UpArgs<T> a) {
+  k_up_body<T, D, FIN>(a, (int)blockIdx.x, (int)gridDim.x, (int)blockIdx.x);
 }
 
 }  // namespace wl

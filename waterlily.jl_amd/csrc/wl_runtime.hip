@@ -258,6 +258,7 @@ struct MG {
     dfree(c_alt);
     dfree(r_alt);
     dfree(arena);
+    dfree(fin_r);
     dfree(tail_img);
     dfree(row_arena);
     for (size_t k = 0; k < lv.size(); ++k) {
@@ -377,6 +378,8 @@ struct MG {
       sg.H = (int64_t)sg.Q * g0.N[1] * g0.N[2];
       se = dalloc<T>(2 * sg.H);
     }
+    r_home = lv[0].r;
+    if (D == 2 && up_ok(0) && perdir == 0 && !use_graphs && !smooth4_ok() && !use_gs_pair && !use_gs_dbl) fin_r = dalloc<T>(lv[0].g.n);
     if (smooth4_ok()) {
       r_alt = dalloc<T>(lv[0].g.n);
       static bool sm_attr = false;  // k_smooth4's LDS ring exceeds the default 64 KB
@@ -901,26 +904,81 @@ struct MG {
     ej_written = true;
     finish_sum(nb, 1, fmode);
   }
-  // Vcycle! (src/MultiLevelPoisson.jl:88-101) from the state "ϵ(0) = r·iD"
-  void vcycle(const T* w) {
+  // Vcycle! (src/MultiLevelPoisson.jl:88-101) from the state "ϵ(0) = r·iD"; with fin the finest
+  // level's smooth! too, where k_up does it (true is returned then)
+  bool vcycle(const T* w, bool fin = false) {
     const int Lm = (int)lv.size() - 1;
     bool in_lds = false;
     const int Lt = tail_start(&in_lds);
     const int down_end = Lt > 0 ? Lt : Lm;
     for (int l = 0; l < down_end; ++l) restrict_level(l);  // down-leg: Jacobi! + restrict! + fill!
     if (Lt > 0) launch_tail(Lt, in_lds, w);  // levels Lt..Lm, through smooth!(Lt)
+    bool done = Lt > 0;  // the coarse level's smooth! and increment! are done
     for (int c = Lt > 0 ? Lt : Lm; c >= 1; --c) {  // up-leg: smooth!(coarse), prolongate! + increment!(fine)
-      if (!(Lt > 0 && c == Lt)) {
+      bool fold = false;
+      if (!done) {
         gs_sweeps(c);
-        if (fold_coarse_inc) {  // smooth!'s increment!(c) formed inside the prolongation
-          prolong_level(c, w, true);
-          continue;
-        }
-        increment(c, w, false);
+        if (fold_coarse_inc) fold = true;  // smooth!'s increment!(c) formed inside the prolongation
+        else increment(c, w, false);
       }
-      prolong_level(c, w);
+      done = false;
+      if (!fold && (c > 1 ? up_ok(c - 1) : fin && fin_ok())) {
+        up_level(c - 1, w, c == 1);
+        done = true;
+      } else {
+        prolong_level(c, w, fold);
+      }
+    }
+    return done;
+  }
+  // k_up in place of the separate launches of a level: a flow's own solver (nobody reads the level's
+  // r and ϵ afterwards), levels below up_cells cells.
+  bool up_ok(int l) const {
+    const Geo& g = lv[l].g;
+    for (int d = 0; d < g.D; ++d) if (g.N[d] < 4) return false;
+    return fold_coarse_inc && use_up && g.n <= up_cells(g.D);
+  }
+  bool use_up = true;
+  static int64_t up_cells(int D) {
+    static int64_t v = [] {
+      const char* e = std::getenv("WL_UP_CELLS");
+      return e ? (int64_t)std::atoll(e) : (int64_t)-1;
+    }();
+    return v >= 0 ? v : (D == 3 ? 100000 : (int64_t)1 << 40);
+  }
+  bool fin_ok() const { return lv[0].g.D == 2 && up_ok(0) && fin_r != nullptr && perdir == 0; }
+  T* fin_r = nullptr;  // the residual buffer k_up writes on the finest level; swapped with lv[0].r
+  T* r_home = nullptr; // lv[0].r between solves
+  void up_level(int l, const T* w, bool fin) {
+    Level<T>& f = lv[l];
+    Level<T>& c = lv[l + 1];
+    UpArgs<T> a{f.g, c.g, f.cmask, perdir, lr(l), f.r, f.x, c.x, w, fin_r, jac(l), B->partial, 0, 0};
+    auto tiles = [](int n, int o) { return (n + o - 1) / o; };
+    const Geo& g = f.g;
+    int64_t nb = 0;
+    ProfScope ps(P, st, fin ? "up_fin" : "up", l,
+                 (double)sizeof(T) * ((fin ? 5 : 3) * ncells_inside(g) + ncells_inside(c.g)));
+#define WL_UP(DD, FF)                                                                                       \
+  do {                                                                                                      \
+    using U = UpTile<DD, FF>;                                                                               \
+    const size_t up_bytes = up_lds<T, DD, FF>();                                                            \
+    a.ntx = tiles(g.N[0] - 2, U::OX);                                                                       \
+    a.nty = tiles(g.N[1] - 2, U::OY);                                                                       \
+    nb = (int64_t)a.ntx * a.nty * (DD == 3 ? tiles(g.N[2] - 2, U::OZ) : 1);                                 \
+    if (FF && nb > B->npartial) throw WlErr(WL_EINVAL, "k_up: more blocks than partial slots");             \
+    hipLaunchKernelGGL((k_up<T, DD, FF>), dim3((unsigned)nb), dim3(U::THREADS), up_bytes, st, a);           \
+  } while (0)
+    if (g.D == 3) WL_UP(3, false);
+    else if (fin) WL_UP(2, true);
+    else WL_UP(2, false);
+#undef WL_UP
+    KCK();
+    if (fin) {
+      std::swap(f.r, fin_r);
+      fin_blocks = nb;
     }
   }
+  int64_t fin_blocks = 0;
   // Jacobi! (ω = 1) on level l, restrict! to l+1 and fill!(x, 0) there (src/MultiLevelPoisson.jl:92-94)
   void restrict_level(int l) {
     Level<T>& f = lv[l];
@@ -1098,7 +1156,11 @@ struct MG {
       smooth4(w, 3);  // L₂, then the ω update in the same single-block finish
       return;
     }
-    vcycle(w);
+    if (vcycle(w, true)) {
+      ej_written = true;
+      finish_sum(fin_blocks, 1, 3);
+      return;
+    }
     gs_sweeps(0);
     increment(0, w, true, 3);  // L₂, then the ω update in the same single-block finish
   }
@@ -1162,6 +1224,7 @@ struct MG {
         break;
       }
     }
+    if (fin_r && lv[0].r != r_home) std::swap(lv[0].r, fin_r);  // (its values are not read again)
     perbc(lv[0].g, lv[0].x);
     return n;
   }
