@@ -1,6 +1,6 @@
-"""The coarse levels of a flow's V-cycle on the GPU: the single-workgroup tail (k_mg_tail_fast and
-its general form) and the fused up-leg of a level (k_up), bit for bit against the oracle at the
-sizes where their tiles and thread maps end."""
+"""A flow's V-cycle on the GPU: the single-workgroup tail (k_mg_tail_fast and its general form), the
+fused up-leg of a level (k_up) and the lean passes of large 3D levels (k_lean_*), bit for bit
+against the oracle at the sizes where their tiles and thread maps end."""
 import os
 
 import numpy as np
@@ -31,12 +31,17 @@ CASES = [
     # periodic in one or every direction, exit
     ((64, 48), dict(perdir=(2,))), ((40, 32, 24), dict(perdir=(1, 2, 3))), ((48, 32, 24), dict(perdir=(3,))),
     ((72, 40), dict(exit_bc=True)), ((48, 24, 32), dict(exit_bc=True)),
+    # the lean passes on one level, on two; rows of less and more than a wave's pairs; with exit
+    ((128, 40, 40), dict(lean=True)), ((144, 96, 80), dict(lean=True)), ((264, 56, 56), dict(lean=True)),
+    ((96, 88, 56), dict(lean=True, exit_bc=True)),
 ]
 
 
 @pytest.mark.parametrize("T", [np.float32, np.float64])
 @pytest.mark.parametrize("n,kw", CASES, ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else "".join(v))
-def test_flow_steps_bitwise(wl, n, kw, T):
+def test_flow_steps_bitwise(wl, n, kw, T, monkeypatch):
+    if kw.get("lean"):
+        monkeypatch.setenv("WL_LEAN", "2")  # at every size
     if T is np.float64 and kw.get("exit_bc"):
         pytest.skip("the exit plane's sums are Float64 on both sides, in orders of their own: Float64 shows it")
     print("case: coarse levels", n, kw, T.__name__, flush=True)
@@ -57,3 +62,29 @@ def test_flow_steps_bitwise(wl, n, kw, T):
         assert sim.pois.n == o.n, k
         for name in ("u", "p"):
             assert np.array_equal(sim.flow.get(name), o.flow.get(name)), (k, name)
+
+
+@pytest.mark.parametrize("T", [np.float32, np.float64])
+@pytest.mark.parametrize("how", ["body moves", "no body", "g and itmx 2", "profile"])
+def test_lean_equals_plain(wl, how, T, monkeypatch):
+    """The lean passes against the general ones (WL_LEAN=0) on the same flow: the coefficients' flags
+    and 1/D follow a body that moves along and across the segments' ends, a flow without one has no
+    row that reads them, and a projection cut after two V-cycles leaves the same p and u."""
+    print("case: lean and plain", how, T.__name__, flush=True)
+    n, got = (272, 56, 48), {}
+    for mode in ("0", "2"):
+        monkeypatch.setenv("WL_LEAN", mode)
+        body = None if how == "no body" else wl.Sphere((60.3, 26.0, 24.0), 9)
+        sim = wl.Simulation(n, (1, 0, 0), 18, ν=0.02, body=body, T=T, exitBC=how == "profile",
+                            g=(lambda i, x, t: 0.1 * t) if how == "g and itmx 2" else None)
+        if how == "g and itmx 2":
+            sim.pois.set_solver(itmx=2)
+        sim.flow.profile(how == "profile")
+        got[mode] = []
+        for k in range(4):
+            if how == "body moves":  # its edge passes the end of the first 128 cells
+                sim.body = wl.Sphere((100.0 + 7.5 * k, 12.0 + 4 * k, 40.0 - 6 * k), 9)
+            wl.sim_step(sim, remeasure=how == "body moves")
+            got[mode] += [sim.flow.get("u"), sim.flow.get("p"), list(sim.pois.n)]
+    for a, b in zip(got["0"], got["2"]):
+        assert np.array_equal(a, b)

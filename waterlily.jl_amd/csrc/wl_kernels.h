@@ -1139,7 +1139,8 @@ __device__ __forceinline__ void prolong_cell(const Geo& gf, const Geo& gc, int c
 // ---- residual! (src/Poisson.jl:92-98) fused with mom_project!'s z = div(u) and x .*= dt
 // (src/Flow.jl:225).  xin·scale is written to xout; with FLOW the source z is div(u).
 // EL2: also what k_submean_l2 forms when no mean is subtracted, from the same values over the
-// same tiles: ϵ = r·iD into eout and the block Σr² into partial[pstride + pidx].
+// same tiles: ϵ = r·iD into eout (unless null) and the block Σr² into partial[pstride + pidx].  A
+// projection whose V-cycles form ϵ and x again (k_lean_*) passes null for eout and z, write_x = 0.
 template <class T, bool FLOW, bool EL2 = false>
 __device__ __forceinline__ void k_residual_body(const Geo& g, const ZT& t, const LRows<T>& LR, const T* __restrict__ xin,
                                                   T* __restrict__ xout, T scale, int write_x, T* __restrict__ z,
@@ -1177,12 +1178,12 @@ __device__ __forceinline__ void k_residual_body(const Geo& g, const ZT& t, const
       const T Dg = diag_at<T>(g, L, I);
       const T iD = inv_diag(Dg);
       const T rv = iD == T(0) ? T(0) : zv - mult_nb<T>(g, L, I, Dg, x0, v);
-      if (FLOW) z[I] = zv;
+      if (FLOW && z) z[I] = zv;
       r[I] = rv;
       if (write_x) xout[I] = x0;
       acc += (double)rv;
       if (EL2) {
-        eout[I] = rv * iD;
+        if (eout) eout[I] = rv * iD;
         acc2 += (double)rv * (double)rv;
       }
     }
@@ -1993,6 +1994,10 @@ __global__ void __launch_bounds__(256) k_inc_restrict2(Geo gf, Geo gc, ZT t, LRo
     }
   }
 }
+
+}  // namespace wl
+#include "wl_lean.h"
+namespace wl {
 
 // smooth!(p) of the finest level in one pass (src/Poisson.jl:141-148 with GaussSeidelRB!, 3D, no
 // periodic directions, even inside x extent and even last ghosted extent): ϵ = r·iD, the four

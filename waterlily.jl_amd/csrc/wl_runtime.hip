@@ -228,6 +228,11 @@ struct Level {
   uint8_t* lrow = nullptr;
   bool lrow_ok = false;  // flags match the current L
   T lc[3] = {1, 1, 1};   // the level's uniform face value per component
+  // a level the lean passes can run (k_lean_*): the residual after the prolongation, 1/D, and on a
+  // coarse level the colour-split ϵ (the finest level's is MG::se)
+  T *r2 = nullptr, *iD = nullptr, *se = nullptr;
+  uint8_t* lseg = nullptr;  // per row and 128 cells: bits, uniform, fast (k_seg_*)
+  SplitG sg{0, 0};
 };
 
 struct Bufs {  // reduction scratch shared by a handle
@@ -265,6 +270,10 @@ struct MG {
       Level<T>& l = lv[k];
       dfree(l.e2);
       dfree(l.ej);
+      dfree(l.r2);
+      dfree(l.iD);
+      dfree(l.lseg);
+      dfree(l.se);
       if (k > 0) continue;  // the coarse levels' arrays lie in the arenas
       if (l.ownL) dfree(l.L);
       if (l.ownx) dfree(l.x);
@@ -341,6 +350,8 @@ struct MG {
       use_smooth4 = e4 && std::atoi(e4) != 0;
       const char* e8 = std::getenv("WL_SPLIT");
       use_split = !e8 || std::atoi(e8) != 0;
+      const char* e9 = std::getenv("WL_LEAN");
+      lean_sizes = e9 ? std::atoi(e9) : 1;
     }
     lv.push_back(l0);
     if (!multilevel) return;
@@ -377,6 +388,22 @@ struct MG {
       sg.Q = g0.N[0] / 2 + 1;
       sg.H = (int64_t)sg.Q * g0.N[1] * g0.N[2];
       se = dalloc<T>(2 * sg.H);
+      lv[0].sg = sg;
+      // the lean passes' buffers (two fields and the coarser levels') only where there is plenty of room,
+      // so that what fits without them still does
+      size_t room = 0, card = 0;
+      HIPCK(hipMemGetInfo(&room, &card));
+      const bool plenty = (double)room > 40.0 * (double)(g0.n * (int64_t)sizeof(T));
+      for (int l = 0; l < (int)lv.size() && plenty && lean_level(l); ++l) {
+        Level<T>& p = lv[l];
+        p.r2 = dalloc<T>(p.g.n);
+        p.iD = dalloc<T>(p.g.n);
+        p.lseg = dalloc<uint8_t>(3 * (int64_t)lean_nseg(p.g) * p.g.N[1] * p.g.N[2]);
+        if (l == 0) continue;
+        p.sg.Q = p.g.N[0] / 2 + 1;
+        p.sg.H = (int64_t)p.sg.Q * p.g.N[1] * p.g.N[2];
+        p.se = dalloc<T>(2 * p.sg.H);
+      }
     }
     r_home = lv[0].r;
     if (D == 2 && up_ok(0) && perdir == 0 && !use_graphs && !smooth4_ok() && !use_gs_pair && !use_gs_dbl) fin_r = dalloc<T>(lv[0].g.n);
@@ -433,6 +460,11 @@ struct MG {
     const int64_t nr = (int64_t)p.g.N[1] * p.g.N[2];
     p.lrow_ok = false;
     if (l == 0) ++lrow_epoch0;
+    if (p.iD) {
+      Box b = box_inside(p.g);
+      hipLaunchKernelGGL(k_diag<T>, grid_of(b), kBlock, 0, st, p.g, b, (const T*)p.L, p.iD, 1);
+      KCK();
+    }
     if (!use_lrows) return;
     hipLaunchKernelGGL(k_lrow_bits<T>, dim3((unsigned)((nr + 3) / 4)), dim3(256), 0, st, p.g, (const T*)p.L,
                        p.lc[0], p.lc[1], p.lc[2], p.lrow);
@@ -440,6 +472,19 @@ struct MG {
     hipLaunchKernelGGL(k_lrow_flags, dim3((unsigned)((nr + 255) / 256)), dim3(256), 0, st, p.g,
                        (const uint8_t*)p.lrow, p.lrow + nr);
     KCK();
+    if (p.iD) {
+      const int ns = lean_nseg(p.g);
+      const int64_t nk = nr * ns;
+      hipLaunchKernelGGL(k_seg_bits<T>, dim3((unsigned)((nk + 3) / 4)), dim3(256), 0, st, p.g, (const T*)p.L, p.lc[0],
+                         p.lc[1], p.lc[2], ns, p.lseg);
+      KCK();
+      hipLaunchKernelGGL(k_seg_uniform, dim3((unsigned)((nk + 255) / 256)), dim3(256), 0, st, p.g, ns,
+                         (const uint8_t*)p.lseg, p.lseg + nk);
+      KCK();
+      hipLaunchKernelGGL(k_seg_fast, dim3((unsigned)((nk + 255) / 256)), dim3(256), 0, st, p.g, ns,
+                         (const uint8_t*)p.lseg + nk, p.lseg + 2 * nk);
+      KCK();
+    }
     p.lrow_ok = true;
   }
   void ensure_lrows() {
@@ -468,14 +513,118 @@ struct MG {
   }
   bool split_ready() const { return se != nullptr && split_ok(); }
   void split_swap() { std::swap(lv[0].e, se); }
-  void split_begin() {
+  // The lean passes (k_lean_*): levels of the colour-split solver that are coarsened in every
+  // direction and too large for k_up, from the size on where a level's fields no longer stay in the
+  // 256 MB last-level cache (below, the plain passes' extra values cost little and an update's 1/D and
+  // flags more).  Step with a static body, plain -> lean, us: FP32 256x128x128 880 -> 851, 320x160x160
+  // 1684 -> 1645, 384x192x192 3133 -> 2880, 512x256x256 7592 -> 6352; FP64 320x160x160 (as many bytes
+  // as FP32 402x201x201) 3442 -> 3081; with a body measured in each step 1314 -> 1329, 2425 -> 2470,
+  // 3614 -> 3521, 8121 -> 7414; 4411 -> 4124.  Coarser levels, under a lean one: at 17 MB 6352 -> 6258,
+  // at 14 MB 5398 -> 5471.
+  bool lean_on = false;  // this projection runs them on every level that has r2
+  bool lean_level(int l) const {
+    bool in_lds = false;
+    const int Lt = tail_start(&in_lds);
+    return lv[l].g.D == 3 && perdir == 0 && fold_coarse_inc && lv[l].cmask == 7 && l + 1 < (int)lv.size() &&
+           (Lt < 0 || l < Lt) && pairs_ok(l) && !up_ok(l) &&
+           (lean_sizes == 2 || (lean_sizes == 1 && lv[l].g.n * (int64_t)sizeof(T) >= (l == 0 ? 40 << 20 : 16 << 20)));
+  }
+  bool lean(int l) const { return lean_on && lv[l].r2 != nullptr; }
+  const T* lean_p = nullptr;  // the projection's p and Δt (x = p·Δt before its first V-cycle)
+  T lean_dt = T(0);
+  LeanL<T> lean_args(int l) const {
+    const Level<T>& p = lv[l];
+    const int ns = lean_nseg(p.g);
+    return lean_l<T>(p.L, p.iD, p.lrow_ok ? p.lseg + 2 * (int64_t)ns * p.g.N[1] * p.g.N[2] : nullptr, ns, p.lc);
+  }
+  // z runs of whole plane pairs (the inside's extents are even: z0 odd, z1 even): 8 planes where that
+  // leaves 8192 blocks, down to 4 (half sweep at 512x256x256 with 4, 8, 16 planes: 89, 77, 78 us,
+  // prolongation 145, 130, 134; at 256x128x128 12.2, 12.3, 14.4 and 23.7, 27.6, 37.5)
+  static ZT lean_zt(const Box& b) {
+    ZT t = make_zt(b);
+    const int nz = b.hi[2] - b.lo[2] + 1;
+    const int64_t zc = (int64_t)nz * t.nbx * t.nby / 8192;
+    t.zc = (int)std::min<int64_t>(8, std::max<int64_t>(4, zc & ~1));
+    return t;
+  }
+  T* lean_eps(int l) const { return l == 0 ? lv[0].e : lv[l].se; }  // lv[0].e: between split_begin and _end
+  void restrict_lean(int l) {
+    Level<T>& f = lv[l];
+    Level<T>& c = lv[l + 1];
+    bool in_lds = false;
+    const int Lt = tail_start(&in_lds);
+    const bool ce = !(lean(l + 1) || (l + 1 == Lt && in_lds && tail_fast(Lt)));
+    ProfScope ps(P, st, "inc_restrict", l, (double)sizeof(T) * (ncells_inside(f.g) + (ce ? 3 : 1) * ncells_inside(c.g)));
+    ZT bc = make_zt(box_inside(c.g), tgt_rp());
+    bc.sx = 32;
+    bc.nbx = (bc.b.hi[0] - bc.b.lo[0] + 32) / 32;
+    // 4 coarse planes per tile (2, 8, 16: 88, 79, 80 us against 75 at 512x256x256; 15.7, 17.6, 25
+    // against 15.1 at 256x128x128)
+    bc.zc = 4;
+    if (ce)
+      hipLaunchKernelGGL((k_lean_restrict<T, true>), zt_grid(bc), kBlock, 0, st, f.g, c.g, bc, lean_args(l),
+                         (const T*)f.r, lr(l + 1), c.r, c.x, c.e);
+    else
+      hipLaunchKernelGGL((k_lean_restrict<T, false>), zt_grid(bc), kBlock, 0, st, f.g, c.g, bc, lean_args(l),
+                         (const T*)f.r, lr(l + 1), c.r, c.x, c.e);
+    KCK();
+  }
+  // from level c into c − 1; fold: x + ω·ϵ of level c is formed at the cells read
+  void prolong_lean(int c, const T* w, bool fold) {
+    const int l = c - 1;
+    Level<T>& f = lv[l];
+    Level<T>& k = lv[c];
+    ProfScope ps(P, st, "prolong_inc", l,
+                 (double)sizeof(T) * ((l > 0 ? 3 : 2) * ncells_inside(f.g) + (fold ? 2 : 1) * ncells_inside(k.g)));
+    const ZT bp = lean_zt(box_pairs(f.g));
+#define WL_LP(CI, SP, XWV)                                                                                        hipLaunchKernelGGL((k_lean_prolong<T, CI, SP, XWV>), zt_grid(bp), kBlock, 0, st, f.g, k.g, bp, lean_args(l),                         (const T*)f.r, f.r2, f.x, (const T*)k.x, (const T*)(lean(c) ? k.se : k.e), k.sg, w)
+    if (l > 0) {
+      if (!fold) WL_LP(false, false, true); else if (lean(c)) WL_LP(true, true, true); else WL_LP(true, false, true);
+    } else {
+      if (!fold) WL_LP(false, false, false); else if (lean(c)) WL_LP(true, true, false); else WL_LP(true, false, false);
+    }
+#undef WL_LP
+    KCK();
+  }
+  void gs_lean(int l) {
+    Level<T>& p = lv[l];
+    const ZT b = lean_zt(box_pairs(p.g));
+    T* e = lean_eps(l);
+    ProfScope ps(P, st, "gs_half", l, gs_bytes(l), 4);
+    hipLaunchKernelGGL(k_lean_gs_first<T>, zt_grid(b), kBlock, 0, st, p.g, p.sg, b, lean_args(l), (const T*)p.r2, e);
+    KCK();
+    for (int it = 2; it <= 4; ++it) {
+      hipLaunchKernelGGL(k_lean_gs<T>, zt_grid(b), kBlock, 0, st, p.g, p.sg, b, lean_args(l), (const T*)p.r2, e, it);
+      KCK();
+    }
+  }
+  // the finest level's increment!; first: x is still p·Δt
+  void increment_lean(const T* w, bool first, int fmode) {
+    Level<T>& f = lv[0];
+    Level<T>& k = lv[1];
+    const ZT b = lean_zt(box_pairs(f.g));
+    ProfScope ps(P, st, "increment", 0, (double)sizeof(T) * (6 * ncells_inside(f.g) + 2 * ncells_inside(k.g)));
+    const T* xin = first ? lean_p : (const T*)f.x;
+    const T scale = first ? lean_dt : T(1);
+    const bool fold = lean_fold1;
+#define WL_LI(CI, SP)                                                                                                hipLaunchKernelGGL((k_lean_increment<T, CI, SP>), zt_grid(b), kBlock, 0, st, f.g, k.g, b, lean_args(0), f.r,                             (const T*)f.r2, xin, scale, f.x, (const T*)f.e, f.sg, (const T*)k.x,                                              (const T*)(lean(1) ? k.se : k.e), k.sg, w, B->partial)
+    if (!fold) WL_LI(false, false); else if (lean(1)) WL_LI(true, true); else WL_LI(true, false);
+#undef WL_LI
+    KCK();
+    finish_sum(zt_blocks(b), 1, fmode);
+  }
+  bool lean_fold1 = false;  // level 1's x of this V-cycle still lacks its last increment!
+  void split_begin(bool plain) {
     split_swap();
     split_on = true;
+    lean_on = plain && lv[0].r2 != nullptr;
   }
+  int lean_sizes = 1;  // WL_LEAN: 0 none, 1 levels from the sizes of lean_level on, 2 every level it can be
   void split_end() {
     if (!split_on) return;
     split_swap();
     split_on = false;
+    lean_on = false;
   }
   // x-pair kernels (k_gs_half2, k_increment2): an even inside x extent, and an even last ghosted
   // extent (half_rangek then reaches every inside cell, which the pair sweep updates); WL_PAIRS=0
@@ -917,7 +1066,7 @@ struct MG {
     for (int c = Lt > 0 ? Lt : Lm; c >= 1; --c) {  // up-leg: smooth!(coarse), prolongate! + increment!(fine)
       bool fold = false;
       if (!done) {
-        gs_sweeps(c);
+        if (lean(c)) gs_lean(c); else gs_sweeps(c);
         if (fold_coarse_inc) fold = true;  // smooth!'s increment!(c) formed inside the prolongation
         else increment(c, w, false);
       }
@@ -925,6 +1074,9 @@ struct MG {
       if (!fold && (c > 1 ? up_ok(c - 1) : fin && fin_ok())) {
         up_level(c - 1, w, c == 1);
         done = true;
+      } else if (lean(c - 1)) {
+        prolong_lean(c, w, fold);
+        if (c == 1) lean_fold1 = fold;
       } else {
         prolong_level(c, w, fold);
       }
@@ -981,6 +1133,10 @@ struct MG {
   int64_t fin_blocks = 0;
   // Jacobi! (ω = 1) on level l, restrict! to l+1 and fill!(x, 0) there (src/MultiLevelPoisson.jl:92-94)
   void restrict_level(int l) {
+    if (lean(l)) {
+      restrict_lean(l);
+      return;
+    }
     Level<T>& f = lv[l];
     Level<T>& c = lv[l + 1];
     T* fe = jac(l);
@@ -996,6 +1152,7 @@ struct MG {
       const int64_t per = (int64_t)bc.nbx * bc.nby;
       const int nz = bc.b.hi[2] - bc.b.lo[2] + 1;
       bc.zc = (int)std::min<int64_t>(32, std::max<int64_t>(1, (int64_t)nz * per / tgt_rp()));
+    if (std::getenv("R_ZC")) bc.zc = std::atoi(std::getenv("R_ZC"));
       if (f.g.D == 3)
         hipLaunchKernelGGL((k_inc_restrict2<T, 3>), zt_grid(bc), kBlock, 0, st, f.g, c.g, bc, lr(l), f.r, f.x,
                            (const T*)fe, lr(l + 1), c.r, c.x, c.e);
@@ -1082,7 +1239,7 @@ struct MG {
       MG* m;
       ~SplitScope() { if (m) m->split_end(); }
     } split_scope{sp ? this : nullptr};
-    if (sp) split_begin();
+    if (sp) split_begin(true);
     Level<T>& f = lv[0];
     Level<T>& c = lv[1];
     T* bufs[6] = {f.e, f.r, f.x, c.e, c.r, c.x};
@@ -1119,7 +1276,7 @@ struct MG {
       int pick = 0;
       for (int cnd : cands) {
         zt_gs = cnd;
-        const float ms = timed([&] { gs_sweeps(0); });
+        const float ms = timed([&] { if (lean(0)) gs_lean(0); else gs_sweeps(0); });
         if (ms < best) { best = ms; pick = cnd; }
       }
       zt_gs = pick;
@@ -1127,7 +1284,10 @@ struct MG {
       pick = 0;
       for (int cnd : cands) {
         zt_rp = cnd;
-        const float ms = timed([&] { restrict_level(0); prolong_level(1, w); });
+        const float ms = timed([&] {
+          restrict_level(0);
+          if (lean(0)) prolong_lean(1, w, lean(1)); else prolong_level(1, w);
+        });
         if (ms < best) { best = ms; pick = cnd; }
       }
       zt_rp = pick;
@@ -1148,7 +1308,7 @@ struct MG {
   // (src/MultiLevelPoisson.jl:113-121).  `first`: ϵ(0) = r·iD is already set by residual!.
   void iteration(bool first) {
     const T* w = (const T*)B->tsc + 3;
-    if (!first && !ej_written) eps_init(0);
+    if (!first && !ej_written && !lean_on) eps_init(0);
     if (smooth4_ok()) {
       skip_eps0 = true;  // the level-0 prolongation leaves ϵ to k_smooth4
       vcycle(w);
@@ -1159,6 +1319,11 @@ struct MG {
     if (vcycle(w, true)) {
       ej_written = true;
       finish_sum(fin_blocks, 1, 3);
+      return;
+    }
+    if (lean(0)) {
+      gs_lean(0);
+      increment_lean(w, first, 3);
       return;
     }
     gs_sweeps(0);
@@ -1875,7 +2040,7 @@ struct FlowT : FlowBase {
         MG<T>* m;
         ~SplitScope() { if (m) m->split_end(); }
       } split_scope{split ? &mg : nullptr};
-      if (split) mg.split_begin();
+      if (split) mg.split_begin(false);
       nit = mg.mixed_loop(tol, itmx, &r2hist);
     }
     hipLaunchKernelGGL(k_round_x<T>, zt_grid(bi), kBlock, 0, st, g, bi, (const double*)mg.x64[mg.x64cur], xw);
@@ -1967,15 +2132,21 @@ struct FlowT : FlowBase {
       MG<T>* m;
       ~SplitScope() { if (m) m->split_end(); }
     } split_scope{split ? &mg : nullptr};
-    if (split) mg.split_begin();
+    if (split) mg.split_begin(true);
+    if (itmx <= 0) mg.lean_on = false;  // no V-cycle would write x
+    const bool lean = mg.lean_on;
+    mg.lean_p = p;
+    mg.lean_dt = dt;
     Level<T>& l0 = mg.lv[0];
     ZT bi = zt_inside(g);
     const int64_t nb = zt_blocks(bi);
     {
-    // with ϵ = r·iD and the Σr² partials (at partial + nb) as submean would form them unflagged
-    ProfScope ps(&prof, st, "residual", 0, (double)sizeof(T) * (D + 5) * ncells_inside(g));
+    // with ϵ = r·iD and the Σr² partials (at partial + nb) as submean would form them unflagged; the
+    // lean V-cycles need neither ϵ nor x, and div(u) is kept only where a udf! may read σ
+    ProfScope ps(&prof, st, "residual", 0, (double)sizeof(T) * (D + (lean ? 2 : 5)) * ncells_inside(g));
     hipLaunchKernelGGL((k_residual<T, true, true>), zt_grid(bi), kBlock, 0, st, g, bi, mg.lr(0), (const T*)p, xw, dt,
-                       1, sigma, (const T*)u, l0.r, B.partial, mg.jac(0), nb);
+                       lean ? 0 : 1, lean && !udf ? (T*)nullptr : sigma, (const T*)u, l0.r, B.partial,
+                       lean ? (T*)nullptr : mg.jac(0), nb);
     KCK();
     }
     mg.perbc(g, xw);
