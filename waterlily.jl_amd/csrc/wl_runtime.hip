@@ -7,6 +7,7 @@
 #include <cstdio>
 #include <cstring>
 #include <cmath>
+#include <chrono>
 #include <string>
 #include <vector>
 #include <memory>
@@ -241,8 +242,31 @@ struct Bufs {  // reduction scratch shared by a handle
   double* dsc = nullptr;   // device doubles
   void* tsc = nullptr;     // device T scalars
   double* hsc = nullptr;   // pinned host doubles
-  void* htsc = nullptr;    // pinned host T
+  double* host = nullptr;  // coherent pinned host doubles (HostSlot): what the host waits for
 };
+
+// Wait for a value that a kernel of stream st posts (host_post).  Read without the copy and the
+// synchronisation's own packets for the first 200 us, then the stream is waited for, which also
+// reports a failed launch.
+static void host_unset(const Bufs& B, int slot) {
+  __atomic_store_n((unsigned long long*)B.host + slot, HOST_UNSET, __ATOMIC_RELEASE);
+}
+static double host_wait(const Bufs& B, int slot, hipStream_t st) {
+  const unsigned long long* p = (const unsigned long long*)B.host + slot;
+  const auto t0 = std::chrono::steady_clock::now();
+  unsigned long long v;
+  while ((v = __atomic_load_n(p, __ATOMIC_ACQUIRE)) == HOST_UNSET) {
+    __builtin_ia32_pause();
+    if (std::chrono::steady_clock::now() - t0 < std::chrono::microseconds(200)) continue;
+    HIPCK(hipStreamSynchronize(st));
+    v = __atomic_load_n(p, __ATOMIC_ACQUIRE);
+    if (v == HOST_UNSET) throw WlErr(WL_EHIP, "internal: a launch ended without the value the host waits for");
+    break;
+  }
+  double d;
+  std::memcpy(&d, &v, sizeof d);
+  return d;
+}
 
 template <class T>
 struct MG {
@@ -670,7 +694,7 @@ struct MG {
   // the partials start at B->partial + poff
   double finish_sum(int64_t np, int slot, int mode = 0, double ninside = 1, int64_t poff = 0) {
     hipLaunchKernelGGL(k_finish_sum<T>, dim3(1), dim3(1024), 0, st, (const double*)B->partial + poff, np, B->dsc + slot,
-                       (T*)B->tsc, mode, ninside, B->dsc);
+                       (T*)B->tsc, mode, ninside, B->dsc, B->host);
     KCK();
     return 0;
   }
@@ -718,7 +742,7 @@ struct MG {
       hipLaunchKernelGGL(k_submean_l2<T>, zt_grid(b), kBlock, 0, st, p.g, b, lr(0), p.r, jac(0), (const T*)B->tsc,
                          B->partial);
     KCK();
-    finish_sum(nb, 1, init ? 2 : 0, 1, cond ? nb : 0);
+    finish_sum(nb, 1, init ? FIN_INIT : FIN_SUM, 1, cond ? nb : 0);
   }
   static int64_t ninside(const Geo& g) {
     int64_t m = 1;
@@ -1318,7 +1342,7 @@ struct MG {
     }
     if (vcycle(w, true)) {
       ej_written = true;
-      finish_sum(fin_blocks, 1, 3);
+      finish_sum(fin_blocks, 1, FIN_CONTROL);
       return;
     }
     if (lean(0)) {
@@ -1374,12 +1398,11 @@ struct MG {
       if (hist) hist->push_back((double)(T)read_dsc(1));
     }
     while (n < itmx) {
+      host_unset(*B, HOST_R2);
       run_iteration(n == 0);
-      HIPCK(hipMemcpyAsync(B->hsc, B->dsc, 8 * sizeof(double), hipMemcpyDeviceToHost, st));
-      HIPCK(hipStreamSynchronize(st));
-      const T rnew = (T)B->hsc[1];
+      const T rnew = (T)host_wait(*B, HOST_R2, st);
       if (hist) {
-        if (n == 0) hist->push_back(B->hsc[6]);
+        if (n == 0) hist->push_back(B->host[HOST_R2_OLD]);
         hist->push_back((double)rnew);
       }
       n++;
@@ -1555,14 +1578,14 @@ static void alloc_bufs(Bufs& B, int64_t np, size_t tsize) {
   B.tsc = dalloc<double>(8);
   (void)tsize;
   HIPCK(hipHostMalloc((void**)&B.hsc, 8 * sizeof(double), hipHostMallocDefault));
-  HIPCK(hipHostMalloc(&B.htsc, 8 * sizeof(double), hipHostMallocDefault));
+  HIPCK(hipHostMalloc((void**)&B.host, HOST_SLOTS * sizeof(double), hipHostMallocCoherent));
 }
 static void free_bufs(Bufs& B) {
   dfree(B.partial);
   dfree(B.dsc);
   dfree(B.tsc);
   if (B.hsc) (void)hipHostFree(B.hsc);
-  if (B.htsc) (void)hipHostFree(B.htsc);
+  if (B.host) (void)hipHostFree(B.host);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1758,9 +1781,9 @@ struct FlowT : FlowBase {
     KCK();
     hipLaunchKernelGGL(k_row_list, dim3(1), dim3(1024), 0, st, g, (const uint8_t*)crows(), rlist, cnt);
     KCK();
-    HIPCK(hipMemcpyAsync(B.htsc, cnt, sizeof(int), hipMemcpyDeviceToHost, st));
+    HIPCK(hipMemcpyAsync(B.hsc, cnt, sizeof(int), hipMemcpyDeviceToHost, st));
     HIPCK(hipStreamSynchronize(st));
-    std::memcpy(&nlist, B.htsc, sizeof(int));
+    std::memcpy(&nlist, B.hsc, sizeof(int));
     crows_ok = true;
     crows_epoch = mg.lrow_epoch0;
   }
@@ -2150,7 +2173,7 @@ struct FlowT : FlowBase {
     KCK();
     }
     mg.perbc(g, xw);
-    mg.finish_sum(nb, 0, 1, (double)MG<T>::ninside(g));
+    mg.finish_sum(nb, 0, FIN_MEAN, (double)MG<T>::ninside(g));
     // without a guess the solver's start state is set in submean's finish (the guess would change
     // Σr²); submean itself runs only where the mean is subtracted
     mg.submean_l2(!use_net, true);
@@ -2189,14 +2212,13 @@ struct FlowT : FlowBase {
     T* tpart = (T*)B.partial;
     {
       ProfScope ps(&prof, st, "cfl", 0, (double)sizeof(T) * (D + 1) * ncells_inside(g));
+      host_unset(B, HOST_MAX);
       hipLaunchKernelGGL(k_cfl<T>, zt_grid(ba), kBlock, 0, st, g, ba, (const T*)u, sigma, tpart);
       KCK();
     }
-    hipLaunchKernelGGL(k_finish_max<T>, dim3(1), dim3(1024), 0, st, (const T*)tpart, nb, (T*)B.tsc + 2);
+    hipLaunchKernelGGL(k_finish_max<T>, dim3(1), dim3(1024), 0, st, (const T*)tpart, nb, B.host);
     KCK();
-    HIPCK(hipMemcpyAsync(B.htsc, (T*)B.tsc + 2, sizeof(T), hipMemcpyDeviceToHost, st));
-    HIPCK(hipStreamSynchronize(st));
-    const T m = ((T*)B.htsc)[0];
+    const T m = (T)host_wait(B, HOST_MAX, st);
     // a non-finite maximum means a NaN or Inf in u (the kernel turns one into +Inf): no Δt
     if (!std::isfinite(m)) return std::numeric_limits<double>::quiet_NaN();
     const T inv = T(1) / (m + T(5) * (T)desc.nu);
