@@ -135,7 +135,7 @@ template <class T>
 __global__ void __launch_bounds__(256) kb_submean(const ALev<T>* __restrict__ A, const BBlk* __restrict__ blk) {
   const BBlk b = blk[blockIdx.x];
   const ALev<T>& a = A[b.sim];
-  k_submean_l2_body<T>(a.g, a.t, a.L, a.r, a.e, a.sdev, a.partial, b.lid, b.pidx);
+  k_submean_l2_body<T>(a.g, a.t, a.L, a.r, a.e, a.sdev[0], a.sdev[1] != T(0), a.partial, b.lid, b.pidx);
 }
 // the mean removal of a member whose residual finish flagged one (|s| > 2eps); the other members'
 // blocks return at once, keeping the ϵ and Σr² partials the residual pass formed
@@ -144,7 +144,7 @@ __global__ void __launch_bounds__(256) kb_submean_cond(const ALev<T>* __restrict
   const BBlk b = blk[blockIdx.x];
   const ALev<T>& a = A[b.sim];
   if (a.sdev[1] == T(0)) return;  // the same for the whole block
-  k_submean_l2_body<T>(a.g, a.t, a.L, a.r, a.e, a.sdev, a.partial, b.lid, b.pidx);
+  k_submean_l2_body<T>(a.g, a.t, a.L, a.r, a.e, a.sdev[0], a.sdev[1] != T(0), a.partial, b.lid, b.pidx);
 }
 template <class T>
 __global__ void __launch_bounds__(256) kb_eps_init(const ALev<T>* __restrict__ A, const BBlk* __restrict__ blk,

@@ -65,5 +65,54 @@ __device__ __forceinline__ void fin_apply(int mode, double s, double* __restrict
   }
 }
 
+__device__ __forceinline__ int fin_tid() { return (int)(threadIdx.x + blockDim.x * threadIdx.y); }
+// Whether this block ends last of nb, with the others' partials (each written by its thread 0 before)
+// visible to all of its threads
+__device__ __forceinline__ bool fin_last(unsigned* cnt, unsigned nb) {
+  __shared__ unsigned last;
+  if (fin_tid() == 0) {
+    __threadfence();
+    last = atomicAdd(cnt, 1u) == nb - 1 ? 1u : 0u;
+    if (last) atomicExch(cnt, 0u);
+  }
+  __syncthreads();
+  const bool l = last != 0u;
+  if (l) __threadfence();
+  return l;
+}
+// N sums Σ partial[k·stride .. k·stride + np) as 1024 threads and block_sum add them (k_finish_sum), by a
+// block of 256: each thread stands for four, whose loads and adds run side by side.  Valid in every
+// thread of the first wave.
+template <int N>
+__device__ __forceinline__ void fin_total(const double* partial, int64_t np, int64_t stride, double* out) {
+  __shared__ double sh[N][16];
+  const int t = fin_tid();
+  double a[N][4];
+#pragma unroll
+  for (int k = 0; k < N; ++k)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) a[k][j] = 0;
+#pragma unroll 2
+  for (int64_t q = t; q < np; q += 1024)
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (q + 256 * j < np) a[k][j] += partial[k * stride + q + 256 * j];
+#pragma unroll
+  for (int k = 0; k < N; ++k)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) a[k][j] = wave_sum(a[k][j]);
+  if ((t & 63) == 0)
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) sh[k][4 * j + (t >> 6)] = a[k][j];
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < N; ++k) out[k] = wave_sum((t & 63) < 16 ? sh[k][t & 15] : 0.0);
+  __syncthreads();
+}
+
 }  // namespace wl
 #endif

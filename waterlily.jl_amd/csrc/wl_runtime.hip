@@ -242,6 +242,7 @@ struct Bufs {  // reduction scratch shared by a handle
   double* dsc = nullptr;   // device doubles
   void* tsc = nullptr;     // device T scalars
   double* hsc = nullptr;   // pinned host doubles
+  unsigned* cnt = nullptr; // blocks of the running launch that have ended (fin_last)
   double* host = nullptr;  // coherent pinned host doubles (HostSlot): what the host waits for
 };
 
@@ -727,22 +728,26 @@ struct MG {
     finish_sum(nb, 0, 1, (double)ninside(p.g));
     submean_l2();
   }
-  // init: also set the solver's start state (ω = 1, r₂ = Σr²), so mg_loop(..., true) skips k_mg_init.
-  // cond: the residual kernel already wrote ϵ and the Σr² partials (at partial + nb) as they are
-  // without a mean subtraction; the kernel redoes them only when the mean is subtracted.
-  void submean_l2(bool init = false, bool cond = false) {
+  void submean_l2() {
+    Level<T>& p = lv[0];
+    ZT b = zt_inside(p.g);
+    ProfScope ps(P, st, "submean_l2", 0, (double)sizeof(T) * 3 * ncells_inside(p.g));
+    hipLaunchKernelGGL(k_submean_l2<T>, zt_grid(b), kBlock, 0, st, p.g, b, lr(0), p.r, jac(0), (const T*)B->tsc,
+                       B->partial);
+    KCK();
+    finish_sum(zt_blocks(b), 1, FIN_SUM);
+  }
+  // After a residual that left ϵ and the Σr² partials (at partial + nb) as they are without a mean
+  // subtraction.  init: also set the solver's start state (ω = 1, r₂ = Σr²), so mg_loop(..., true)
+  // skips k_mg_init.
+  void mean_l2(bool init) {
     Level<T>& p = lv[0];
     ZT b = zt_inside(p.g);
     const int64_t nb = zt_blocks(b);
     ProfScope ps(P, st, "submean_l2", 0, (double)sizeof(T) * 3 * ncells_inside(p.g));
-    if (cond)
-      hipLaunchKernelGGL(k_submean_l2_cond<T>, dim3((unsigned)std::min<int64_t>(nb, 256)), kBlock, 0, st, p.g, b,
-                         lr(0), p.r, jac(0), (const T*)B->tsc, B->partial + nb, (int)nb);
-    else
-      hipLaunchKernelGGL(k_submean_l2<T>, zt_grid(b), kBlock, 0, st, p.g, b, lr(0), p.r, jac(0), (const T*)B->tsc,
-                         B->partial);
+    hipLaunchKernelGGL(k_mean_l2<T>, dim3((unsigned)std::min<int64_t>(nb, 256)), kBlock, 0, st, p.g, b, lr(0), p.r, jac(0),
+                       B->partial, (int)nb, init ? FIN_INIT : FIN_SUM, (double)ninside(p.g), B->dsc, (T*)B->tsc, B->cnt);
     KCK();
-    finish_sum(nb, 1, init ? FIN_INIT : FIN_SUM, 1, cond ? nb : 0);
   }
   static int64_t ninside(const Geo& g) {
     int64_t m = 1;
@@ -1387,7 +1392,7 @@ struct MG {
 
   // solver!(ml) loop (src/MultiLevelPoisson.jl:108-127) after residual!: returns V-cycle count.
   // The host reads Σr² back once per iteration for the stop test, as the reference does.
-  // init_done: submean_l2(true) has already set the start state.
+  // init_done: mean_l2(true) has already set the start state.
   int mg_loop(double tol, int itmx, std::vector<double>* hist, bool init_done = false) {
     if (!init_done) {
       hipLaunchKernelGGL(k_mg_init<T>, dim3(1), dim3(64), 0, st, (const double*)B->dsc, (T*)B->tsc);
@@ -1578,6 +1583,7 @@ static void alloc_bufs(Bufs& B, int64_t np, size_t tsize) {
   B.tsc = dalloc<double>(8);
   (void)tsize;
   HIPCK(hipHostMalloc((void**)&B.hsc, 8 * sizeof(double), hipHostMallocDefault));
+  B.cnt = dalloc<unsigned>(1);
   HIPCK(hipHostMalloc((void**)&B.host, HOST_SLOTS * sizeof(double), hipHostMallocCoherent));
 }
 static void free_bufs(Bufs& B) {
@@ -1585,6 +1591,7 @@ static void free_bufs(Bufs& B) {
   dfree(B.dsc);
   dfree(B.tsc);
   if (B.hsc) (void)hipHostFree(B.hsc);
+  dfree(B.cnt);
   if (B.host) (void)hipHostFree(B.host);
 }
 
@@ -2173,10 +2180,9 @@ struct FlowT : FlowBase {
     KCK();
     }
     mg.perbc(g, xw);
-    mg.finish_sum(nb, 0, FIN_MEAN, (double)MG<T>::ninside(g));
-    // without a guess the solver's start state is set in submean's finish (the guess would change
-    // Σr²); submean itself runs only where the mean is subtracted
-    mg.submean_l2(!use_net, true);
+    // without a guess the solver's start state is set by mean_l2 (the guess would change
+    // Σr²)
+    mg.mean_l2(!use_net);
     if (use_net) warm_guess();
     const int nit = mg.mg_loop(tol, itmx, &r2hist, !use_net);
     if (use_net && (net_flags & WL_WARM_RECORD)) net->record<T>(g, (const T*)xw, st);
