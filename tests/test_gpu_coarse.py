@@ -1,6 +1,8 @@
-"""A flow's V-cycle on the GPU: the single-workgroup tail (k_mg_tail_fast and its general form), the
-fused up-leg of a level (k_up) and the lean passes of large 3D levels (k_lean_*), bit for bit
-against the oracle at the sizes where their tiles and thread maps end."""
+"""A flow's V-cycle and what it is built from on the GPU: the single-workgroup tail (k_mg_tail_fast
+and its general form), the fused up-leg of a level (k_up), the lean passes of large 3D levels
+(k_lean_*), bit for bit against the oracle at the sizes where their tiles and thread maps end; the
+measured fields (k_measure) and the levels' coefficients (k_restrictL, k_restrictL_chain)."""
+import itertools
 import os
 
 import numpy as np
@@ -88,3 +90,73 @@ def test_lean_equals_plain(wl, how, T, monkeypatch):
             got[mode] += [sim.flow.get("u"), sim.flow.get("p"), list(sim.pois.n)]
     for a, b in zip(got["0"], got["2"]):
         assert np.array_equal(a, b)
+
+
+def bc_fill(a, perdir, value=0):
+    """BC!(a, value) (src/core.jl:200-219) of a vector field without exit, in the reference's loops."""
+    D = a.ndim - 1
+    for i in range(D):
+        v = a[..., i]
+        for j in range(D):
+            def at(k):
+                return tuple(k if q == j else slice(None) for q in range(D))
+            N = a.shape[j]
+            if j + 1 in perdir:
+                v[at(0)], v[at(N - 1)] = v[at(N - 2)], v[at(1)]
+            elif i == j:
+                v[at(0)] = v[at(1)] = v[at(N - 1)] = value
+            else:
+                v[at(0)], v[at(N - 1)] = v[at(1)], v[at(N - 2)]
+
+
+def restrict_l(fine, perdir):
+    """restrictL (src/MultiLevelPoisson.jl:20-26,42-48) with its BC!, sums in the reference's order."""
+    D = fine.ndim - 1
+    cm = [N % 2 == 0 and N > 4 for N in fine.shape[:D]]
+    Nc = [1 + N // 2 if c else N for N, c in zip(fine.shape[:D], cm)]
+    out = np.zeros(Nc + [D], dtype=fine.dtype)
+    inner = tuple(slice(1, -1) for _ in range(D))
+    for i in range(D):
+        f = fine[inner + (i,)]
+        steps = [(0,) if j == i or not cm[j] else (0, 1) for j in range(D)]
+        parts = [p[::-1] for p in itertools.product(*steps[::-1])]  # z slowest, x fastest
+        s = np.zeros([N - 2 for N in Nc], dtype=fine.dtype)
+        for p in parts:
+            s = s + f[tuple(slice(p[j], None, 2 if cm[j] else None) for j in range(D))]
+        out[inner + (i,)] = s / fine.dtype.type(2) if cm[i] else s
+    bc_fill(out, perdir)
+    return out
+
+
+@pytest.mark.parametrize("T", [np.float32, np.float64])
+@pytest.mark.parametrize("n,perdir", [((64, 48), ()), ((136, 72), (2,)), ((64, 33), ()), ((40, 32, 24), ()),
+                                      ((48, 40, 32), (1, 3)), ((32, 16, 17), ())],
+                         ids=lambda v: "x".join(map(str, v)) or "-")
+def test_measured_fields_and_levels(wl, n, perdir, T):
+    """measure! in one pass: its ghosts are BC!'s bit for bit, μ₁ and V 0 there, and the step uses the
+    same row flags as after an upload of the same fields; update!: every level's L is restrictL's with
+    its BC!.  The body reaches the walls."""
+    print("case: measured fields and levels", n, perdir, T.__name__, flush=True)
+    D, R = len(n), min(n) / 4
+    U = (1,) + (0,) * (D - 1)
+    body = wl.Sphere((3.3,) + tuple(v - 4.4 for v in n[1:]), R)
+    a, b = (wl.Simulation(n, U, 2 * R, ν=0.05, body=body, T=T, perdir=perdir) for _ in range(2))
+    mu0, mu1, V = (a.flow.get(k) for k in ("mu0", "mu1", "V"))
+    ref = mu0.copy()
+    bc_fill(ref, perdir)
+    assert np.array_equal(mu0, ref)
+    ghost = np.ones(mu0.shape[:-1], bool)
+    ghost[tuple(slice(1, -1) for _ in range(D))] = False
+    assert not mu1[ghost].any() and not V.any()
+    for name in ("mu0", "mu1", "V"):
+        b.flow.set(name, b.flow.get(name))
+    b.pois.update()
+    for s in (a, b):
+        wl.sim_step(s, remeasure=False)
+    for name in ("u", "p"):
+        assert np.array_equal(a.flow.get(name), b.flow.get(name)), name
+    ml = wl.MultiLevelPoisson(np.zeros(mu0.shape[:-1], T), mu0, np.zeros(mu0.shape[:-1], T), perdir=perdir)
+    L, l = mu0, 0
+    while l + 1 < len(ml.levels):
+        L, l = restrict_l(L, perdir), l + 1
+        assert np.array_equal(ml.get("L", l), L), l

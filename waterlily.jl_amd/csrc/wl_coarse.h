@@ -419,7 +419,7 @@ __global__ void __launch_bounds__(1024) k_mg_tail_lds(TailDesc<T> d, const T* __
 // to form D and 1/D).  So a thread owns the same pair for a whole visit of a level and keeps its
 // coefficients, residual and x in registers over the four half sweeps; the LDS carries only what
 // other threads read (ϵ, the residuals a restriction sums, the coarse x); the L, D and 1/D of all
-// levels lie in one image in memory, formed when L changes (k_tail_image), so one round of loads
+// levels lie in one image in memory, formed when L changes (k_level_tables), so one round of loads
 // brings them in.
 struct TailLv {           // one level; built on the host, read with scalar loads
   int N0, N1, N2;
@@ -438,20 +438,6 @@ struct TailFast {
   TailLv lv[TAIL_MAX_LEVELS];
 };
 constexpr int TAIL_FAST_PAIRS = 1024, TAIL_WAVE_PAIRS = 64;
-// L, D and 1/D of one level into the image: D and 1/D on inside as set_diag! forms them
-// (src/Poisson.jl:43-46), 0 on ghosts
-template <class T>
-__global__ void __launch_bounds__(256) k_tail_image(Geo g, const T* __restrict__ L, T* __restrict__ img) {
-  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= g.n) return;
-  for (int i = 0; i < g.D; ++i) img[k + i * g.n] = L[k + i * g.n];
-  const int c[3] = {(int)(k % g.N[0]), (int)((k / g.N[0]) % g.N[1]), (int)(k / g.s[2])};
-  bool in = true;
-  for (int q = 0; q < g.D; ++q) in &= c[q] >= 1 && c[q] <= g.N[q] - 2;
-  const T Dg = in ? diag_at<T>(g, L, k) : T(0);
-  img[k + g.D * g.n] = Dg;
-  img[k + (g.D + 1) * g.n] = in ? inv_diag(Dg) : T(0);
-}
 template <class T, int D>
 __device__ __forceinline__ void k_mg_tail_fast_body(const TailFast<T>& d, const T* __restrict__ wp,
                                                     double (*cg)[TAIL_CG_MAX]) {

@@ -15,7 +15,7 @@ namespace wl {
 // Face coefficients L of a level, with optional uniform-row flags. Away from bodies and walls L is
 // a per-level constant: where rows[y + N1·z] is set, every coefficient the stencils of a cell in
 // the x-row (y, z) read is c[i], except the wall faces x = 1 and x = N0-1 of component 0, which
-// are 0 (the flags are built by comparing bit patterns, k_lrow_bits/k_lrow_flags). Such rows form
+// are 0 (the flags are built by comparing bit patterns, k_level_tables). Such rows form
 // the coefficients instead of loading them: same values, same arithmetic, no L traffic.
 template <class T>
 struct LRows {
@@ -660,11 +660,11 @@ __global__ void __launch_bounds__(256) k_conv_rows(Geo g, const uint8_t* __restr
   crows[r] = (uint8_t)((v ? 1 : 0) | (fz ? 2 : 0) | (b ? 4 : 0) | (lu ? 8 : 0) | (fz && !nb ? 16 : 0));
 }
 // The inside rows of crows without bit 1, in increasing row order, into rlist, and their number
-// into *cnt: one 1024-thread block, 1024 rows per pass, each row's place from a block-wide prefix
+// to the host: one 1024-thread block, 1024 rows per pass, each row's place from a block-wide prefix
 // count (wave ballots, then the waves' totals in LDS).  In row order, the rows k_bdim2_rows
 // does next to each other share their neighbour rows in the cache.
 __global__ void __launch_bounds__(1024) k_row_list(Geo g, const uint8_t* __restrict__ crows, int* __restrict__ rlist,
-                                                   int* __restrict__ cnt) {
+                                                   double* __restrict__ host) {
   __shared__ int wsum[16];
   const int64_t nr = (int64_t)g.N[1] * g.N[2];
   const int tid = (int)threadIdx.x, lane = tid & 63, wv = tid >> 6, nw = (int)blockDim.x >> 6;
@@ -689,7 +689,7 @@ __global__ void __launch_bounds__(1024) k_row_list(Geo g, const uint8_t* __restr
     base += tot;
     __syncthreads();  // wsum is rewritten by the next pass
   }
-  if (tid == 0) cnt[0] = base;
+  if (tid == 0) host_post(host, HOST_ROWS, (double)base);
 }
 // the x = N0-1 plane of component 0 (every y, z), from a to b: the exit plane that BC! keeps
 // under exitBC (src/core.jl:212)
@@ -725,44 +725,6 @@ __global__ void __launch_bounds__(256) k_scale_u(Geo g, Box b, T* __restrict__ u
   if (!box_cell(b, i, j, k)) return;
   const int64_t I = at(g, i, j, k);
   for (int c = 0; c < g.D; ++c) u[I + c * g.n] = u[I + c * g.n] * s;
-}
-
-// Uniform-row flags of a level's face coefficients (LRows). Pass 1, one wavefront per x-row
-// (y, z): bit 0 = component 0 over x = 1..N0-1 is c0, except 0 at x = 1 and x = N0-1; bit 1 =
-// component 1 over x = 1..N0-2 is c1; bit 2 = component 2 likewise (compared bit for bit).
-template <class T>
-__global__ void __launch_bounds__(256) k_lrow_bits(Geo g, const T* __restrict__ L, T c0, T c1, T c2,
-                                                   uint8_t* __restrict__ bits) {
-  const int64_t row = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  if (row >= (int64_t)g.N[1] * g.N[2]) return;  // uniform over the wavefront
-  const int y = (int)(row % g.N[1]), z = (int)(row / g.N[1]);
-  const int64_t base = at(g, 0, y, z);
-  bool ok0 = true, ok1 = true, ok2 = true;
-  for (int x = 1 + lane; x <= g.N[0] - 1; x += 64) {
-    ok0 &= same_bits(L[base + x], (x == 1 || x == g.N[0] - 1) ? T(0) : c0);
-    if (x <= g.N[0] - 2) {
-      ok1 &= same_bits(L[base + x + g.n], c1);
-      if (g.D == 3) ok2 &= same_bits(L[base + x + 2 * g.n], c2);
-    }
-  }
-  const bool a0 = __all(ok0), a1 = __all(ok1), a2 = __all(ok2);
-  if (lane == 0) bits[row] = (uint8_t)(a0 | (a1 << 1) | (a2 << 2));
-}
-// Pass 2: a row is uniform when it is an inside row, its own bits are all set, and the rows of
-// its upper y and z neighbours (whose faces the stencils read) have components 1 and 2 uniform.
-__global__ void __launch_bounds__(256) k_lrow_flags(Geo g, const uint8_t* __restrict__ bits,
-                                                    uint8_t* __restrict__ rows) {
-  const int64_t row = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (row >= (int64_t)g.N[1] * g.N[2]) return;
-  const int y = (int)(row % g.N[1]), z = (int)(row / g.N[1]);
-  bool f = y >= 1 && y <= g.N[1] - 2 && (g.D == 2 || (z >= 1 && z <= g.N[2] - 2));
-  if (f) {
-    const int b = bits[row];
-    f = (b & 1) && (b & 2) && (bits[row + 1] & 2);
-    if (g.D == 3) f = f && (b & 4) && (bits[row + g.N[1]] & 4);
-  }
-  rows[row] = f ? 1 : 0;
 }
 
 // rows[y + N1·z] = 1 where some μ₁ component of the x-row is nonzero, vrows[y + N1·z] = 1 where
@@ -1237,8 +1199,8 @@ __global__ void __launch_bounds__(256) k_submean_l2(Geo g, ZT t, LRows<T> LR, T*
 // FIN_INIT the solver's start.  Every block adds up Σr by itself, so where the mean is subtracted this
 // launch goes on with it: each block walks the blocks b = blockIdx.x + k·gridDim.x of the nb-block
 // launch above (same tiles, same partial slots), and the one that ends last adds up the new Σr².
-// One launch for the three that add, subtract where flagged, and add again: 8 -> 4 us at 64x64,
-// 14 -> 6 us at 256x128x128.
+// One launch for the three that add, subtract where flagged, and add again: 8 -> 3.6 us at 192x128,
+// 14 -> 10 us at 256x128x128.
 template <class T>
 __global__ void __launch_bounds__(256) k_mean_l2(Geo g, ZT t, LRows<T> LR, T* __restrict__ r, T* __restrict__ e,
                                                  double* partial, int nb, int mode, double ninside, double* dsc, T* st,
@@ -2644,26 +2606,126 @@ __global__ void __launch_bounds__(256) k_diag(Geo g, Box b, const T* __restrict_
   const T Dg = diag_at(g, L, I);
   Dout[I] = inv ? inv_diag(Dg) : Dg;
 }
-// restrictL (src/MultiLevelPoisson.jl:20-26,42-48): coarse face coefficients
+// Uniform-row flags of several levels in one launch, and the coarse tail's images (update!): blocks
+// blk0 .. of a level take four rows each, one wave per row, then, with an image, 256 cells each.
+// A row is uniform when it is an inside row whose component 0 has its constant over x = 1..N0-1
+// (0 on the wall faces 1 and N0-1), and component 1 over x = 1..N0-2 of the row and of its upper y
+// neighbour, component 2 of the row and of its upper z neighbour (the faces the stencils read), bit
+// for bit.  A row's neighbours are read again rather than their flags by a second launch: a
+// 1024x512 hierarchy took 26 launches of 2 to 9 us, now one of 10.
+constexpr int TAB_MAX = 24;
 template <class T>
-__global__ void __launch_bounds__(256) k_restrictL(Geo gf, Geo gc, Box bc, int cm, const T* __restrict__ Lf,
+struct TabLv {
+  Geo g;
+  const T* L;
+  T c[3];
+  uint8_t* rows;
+  T* img;    // L, D and 1/D of a level of the fast tail; nullptr: none
+  int blk0;  // the level's first block
+};
+template <class T>
+struct Tables {
+  int n;
+  TabLv<T> lv[TAB_MAX];
+};
+// L, D and 1/D of cell k into the image: D and 1/D on inside as set_diag! forms them
+// (src/Poisson.jl:43-46), 0 on ghosts
+template <class T>
+__device__ __forceinline__ void tail_image_cell(const Geo& g, const T* __restrict__ L, T* __restrict__ img, int64_t k) {
+  if (k >= g.n) return;
+  for (int i = 0; i < g.D; ++i) img[k + i * g.n] = L[k + i * g.n];
+  const int c[3] = {(int)(k % g.N[0]), (int)((k / g.N[0]) % g.N[1]), (int)(k / g.s[2])};
+  bool in = true;
+  for (int q = 0; q < g.D; ++q) in &= c[q] >= 1 && c[q] <= g.N[q] - 2;
+  const T Dg = in ? diag_at<T>(g, L, k) : T(0);
+  img[k + g.D * g.n] = Dg;
+  img[k + (g.D + 1) * g.n] = in ? inv_diag(Dg) : T(0);
+}
+template <class T>
+__global__ void __launch_bounds__(256) k_level_tables(Tables<T> d) {
+  int l = 0;
+  while (l + 1 < d.n && (int)blockIdx.x >= d.lv[l + 1].blk0) ++l;
+  const TabLv<T>& q = d.lv[l];
+  const Geo& g = q.g;
+  const int64_t nr = (int64_t)g.N[1] * g.N[2];
+  const int b = (int)blockIdx.x - q.blk0, nrb = (int)((nr + 3) >> 2);
+  if (b >= nrb) {
+    tail_image_cell<T>(g, q.L, q.img, (int64_t)(b - nrb) * 256 + threadIdx.x);
+    return;
+  }
+  const int64_t row = (int64_t)b * 4 + (threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  if (row >= nr) return;  // uniform over the wavefront
+  const int y = (int)(row % g.N[1]), z = (int)(row / g.N[1]);
+  const bool inside = y >= 1 && y <= g.N[1] - 2 && (g.D == 2 || (z >= 1 && z <= g.N[2] - 2));
+  bool ok = inside;
+  if (inside) {
+    const T* L0 = q.L + at(g, 0, y, z);
+    const T* L1 = L0 + g.n;
+    const T* L2 = g.D == 3 ? L1 + g.n : L1;
+    const int64_t s2 = g.D == 3 ? g.s[2] : g.s[1];
+    const T c2 = g.D == 3 ? q.c[2] : q.c[1];
+    for (int x = 1 + lane; x <= g.N[0] - 1; x += 64) {
+      ok &= same_bits(L0[x], (x == 1 || x == g.N[0] - 1) ? T(0) : q.c[0]);
+      if (x <= g.N[0] - 2)
+        ok &= same_bits(L1[x], q.c[1]) && same_bits(L1[x + g.s[1]], q.c[1]) && same_bits(L2[x], c2) &&
+              same_bits(L2[x + s2], c2);
+    }
+  }
+  if (__all(ok) && lane == 0) q.rows[row] = 1;
+  else if (lane == 0) q.rows[row] = 0;
+}
+// restrictL (src/MultiLevelPoisson.jl:20-26,42-48): coarse face coefficients, and BC!(L, 0) on them: a
+// ghost repeats its inside cell's sum (a BC! launch per level before)
+template <class T>
+__device__ __forceinline__ void restrictL_cell(const Geo& gf, const Geo& gc, int cm, int perdir, const T* Lf, T* Lc,
+                                               const int* c) {
+  for (int i = 0; i < gc.D; ++i) {
+    const bool per = (perdir >> i) & 1;
+    T s = 0;
+    if (per || (c[i] > 1 && c[i] < gc.N[i] - 1)) {
+      int lo[3], hi[3];
+      for (int j = 0; j < 3; ++j) {
+        if (j >= gc.D) { lo[j] = hi[j] = c[j]; continue; }
+        const int m = (j != i || per) ? bc_map(c[j], gc.N[j], (perdir >> j) & 1) : c[j];
+        const bool cj = (cm >> j) & 1;
+        if (j == i) { lo[j] = hi[j] = cj ? 2 * m - 1 : m; }
+        else if (cj) { lo[j] = 2 * m - 1; hi[j] = 2 * m; }
+        else { lo[j] = hi[j] = m; }
+      }
+      for (int k = lo[2]; k <= hi[2]; ++k)
+        for (int j = lo[1]; j <= hi[1]; ++j)
+          for (int q = lo[0]; q <= hi[0]; ++q) s += Lf[at(gf, q, j, k) + i * gf.n];
+      if ((cm >> i) & 1) s = s / T(2);
+    }
+    Lc[at(gc, c[0], c[1], c[2]) + i * gc.n] = s;
+  }
+}
+template <class T>
+__global__ void __launch_bounds__(256) k_restrictL(Geo gf, Geo gc, Box bc, int cm, int perdir, const T* __restrict__ Lf,
                                                    T* __restrict__ Lc) {
   int c[3];
   if (!box_cell(bc, c[0], c[1], c[2])) return;
-  for (int i = 0; i < gc.D; ++i) {
-    int lo[3], hi[3];
-    for (int j = 0; j < 3; ++j) {
-      if (j >= gc.D) { lo[j] = hi[j] = c[j]; continue; }
-      const bool cj = (cm >> j) & 1;
-      if (j == i) { lo[j] = hi[j] = cj ? 2 * c[j] - 1 : c[j]; }
-      else if (cj) { lo[j] = 2 * c[j] - 1; hi[j] = 2 * c[j]; }
-      else { lo[j] = hi[j] = c[j]; }
+  restrictL_cell<T>(gf, gc, cm, perdir, Lf, Lc, c);
+}
+// The same down a chain of small levels, one block: a level takes a few dependent loads, less than
+// the launch it had
+template <class T>
+struct ChainL {
+  int n, perdir;  // g[0], L[0]: the finer level's
+  Geo g[TAB_MAX];
+  T* L[TAB_MAX];
+  int cm[TAB_MAX];
+};
+template <class T>
+__global__ void __launch_bounds__(1024) k_restrictL_chain(ChainL<T> d) {
+  for (int l = 1; l < d.n; ++l) {
+    const Geo& gc = d.g[l];
+    for (int k = (int)threadIdx.x; k < (int)gc.n; k += (int)blockDim.x) {
+      const int c[3] = {k % gc.N[0], (k / gc.N[0]) % gc.N[1], k / (gc.N[0] * gc.N[1])};
+      restrictL_cell<T>(d.g[l - 1], gc, d.cm[l - 1], d.perdir, d.L[l - 1], d.L[l], c);
     }
-    T s = 0;
-    for (int k = lo[2]; k <= hi[2]; ++k)
-      for (int j = lo[1]; j <= hi[1]; ++j)
-        for (int q = lo[0]; q <= hi[0]; ++q) s += Lf[at(gf, q, j, k) + i * gf.n];
-    Lc[at(gc, c[0], c[1], c[2]) + i * gc.n] = ((cm >> i) & 1) ? s / T(2) : s;
+    __syncthreads();  // the block's own writes to L[l], before it reads them
   }
 }
 // pcg! pieces (src/Poisson.jl:166-186)
@@ -2718,38 +2780,69 @@ __global__ void __launch_bounds__(256) k_dot(Geo g, Box b, const T* __restrict__
 // =============================================================================================
 // measure! for analytic bodies (src/Body.jl:28-51,74) and pressure_force (src/Metrics.jl:116-133)
 // =============================================================================================
+// measure! (src/Body.jl:28-51) of analytic bodies in one pass over every cell: σ = sdf on inside, V, μ₀
+// with BC!(μ₀, 0) and μ₁, and the flags of the rows that hold a nonzero μ₁ (zeroed beforehand; the
+// rows of V are +0).  A ghost of μ₀ repeats its inside cell's operations.  Each value is written once;
+// three fills, two passes over the cells, two BC! and the flags' pass over μ₁ and V before.
 template <class T>
-__global__ void __launch_bounds__(256) k_measure_sdf(Geo g, Box b, DBodies bs, T* __restrict__ sigma, T d2) {
-  int c[3];
-  if (!box_cell(b, c[0], c[1], c[2])) return;
-  T x[3] = {T(c[0] + 1) - T(1.5), T(c[1] + 1) - T(1.5), T(c[2] + 1) - T(1.5)};
-  sigma[at(g, c[0], c[1], c[2])] = bodies_sdf_d<T>(bs, g.D, x, d2);
+__device__ __forceinline__ T measure_dist(const Geo& g, const DBodies& bs, T d2, const int* c, T* xc) {
+  for (int k = 0; k < 3; ++k) xc[k] = T(c[k] + 1) - T(1.5);
+  return bodies_sdf_d<T>(bs, g.D, xc, d2);
 }
 template <class T>
-__global__ void __launch_bounds__(256) k_measure_fill(Geo g, Box b, DBodies bs, const T* __restrict__ sigma,
-                                                      T* __restrict__ V, T* __restrict__ mu0, T* __restrict__ mu1,
-                                                      T d2, T eps) {
+__global__ void __launch_bounds__(256) k_measure(Geo g, Box b, DBodies bs, T* __restrict__ sigma, T* __restrict__ V,
+                                                 T* __restrict__ mu0, T* __restrict__ mu1, T d2, T eps, int perdir,
+                                                 uint8_t* __restrict__ rows) {
   int c[3];
   if (!box_cell(b, c[0], c[1], c[2])) return;
   const int D = g.D;
-  const int64_t I = at(g, c[0], c[1], c[2]);
-  const int64_t n = g.n;
-  const T dI = sigma[I];
-  if (dI * dI < d2) {
-    for (int i = 0; i < D; ++i) {
-      T x[3] = {T(c[0] + 1) - T(1.5), T(c[1] + 1) - T(1.5), T(c[2] + 1) - T(1.5)};
-      x[i] = x[i] - T(0.5);
-      T di, ni[3];
-      bodies_measure_d<T>(bs, D, x, d2, di, ni);
-      di = fabs(di) <= T(0.5) ? di : copysign(di, dI);
-      V[I + i * n] = 0;
-      mu0[I + i * n] = mu0_d<T>(di, eps);
-      const T m1 = mu1_d<T>(di, eps);
-      for (int j = 0; j < D; ++j) mu1[I + (i + (int64_t)D * j) * n] = m1 * ni[j];
-    }
-  } else if (dI < T(0)) {
-    for (int i = 0; i < D; ++i) mu0[I + i * n] = 0;
+  const int64_t I = at(g, c[0], c[1], c[2]), n = g.n;
+  bool inside = true;
+  for (int q = 0; q < D; ++q) inside &= c[q] >= 1 && c[q] <= g.N[q] - 2;
+  T x[3], dI = T(0);
+  if (inside) {
+    dI = measure_dist<T>(g, bs, d2, c, x);
+    sigma[I] = dI;
   }
+  const bool near = inside && dI * dI < d2;
+  bool nz = false;
+  for (int i = 0; i < D; ++i) {
+    V[I + i * n] = 0;
+    T di = T(0), ni[3], m1 = T(0), m0 = dI < T(0) ? T(0) : T(1);
+    auto face = [&](const int* m, T dm) {  // the body at component i's face of cell m
+      T xf[3] = {T(m[0] + 1) - T(1.5), T(m[1] + 1) - T(1.5), T(m[2] + 1) - T(1.5)};
+      xf[i] = xf[i] - T(0.5);
+      bodies_measure_d<T>(bs, D, xf, d2, di, ni);
+      di = fabs(di) <= T(0.5) ? di : copysign(di, dm);
+    };
+    if (near) {
+      face(c, dI);
+      m0 = mu0_d<T>(di, eps);
+      m1 = mu1_d<T>(di, eps);
+    }
+    for (int j = 0; j < D; ++j) {
+      const T v = near ? m1 * ni[j] : T(0);
+      mu1[I + (i + (int64_t)D * j) * n] = v;
+      nz |= v != T(0);
+    }
+    const bool per = (perdir >> i) & 1;
+    if (!per && (c[i] <= 1 || c[i] == g.N[i] - 1)) {
+      m0 = T(0);
+    } else if (!inside) {
+      int m[3] = {c[0], c[1], c[2]};
+      for (int q = 0; q < D; ++q)
+        if (q != i || per) m[q] = bc_map(c[q], g.N[q], (perdir >> q) & 1);
+      const T dm = measure_dist<T>(g, bs, d2, m, x);
+      if (dm * dm < d2) {
+        face(m, dm);
+        m0 = mu0_d<T>(di, eps);
+      } else {
+        m0 = dm < T(0) ? T(0) : T(1);
+      }
+    }
+    mu0[I + i * n] = m0;
+  }
+  if (nz) rows[c[1] + (int64_t)g.N[1] * c[2]] = 1;
 }
 template <class T>
 __global__ void __launch_bounds__(256) k_pressure_force(Geo g, Box b, DBodies bs, const T* __restrict__ p,

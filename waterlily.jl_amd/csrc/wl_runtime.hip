@@ -225,7 +225,7 @@ struct Level {
   T* ej = nullptr;
   bool ownL = true, ownx = true, ownz = true;
   int cmask = 0;  // coarsening mask towards the next level
-  // uniform-row flags of L: lrow[0, N1·N2) row bits, lrow[N1·N2, 2·N1·N2) the flags
+  // uniform-row flags of L (k_level_tables)
   uint8_t* lrow = nullptr;
   bool lrow_ok = false;  // flags match the current L
   T lc[3] = {1, 1, 1};   // the level's uniform face value per component
@@ -322,7 +322,7 @@ struct MG {
       int64_t o = 0, ro = 0;
       for (size_t k = lv.size() - 1; k >= 1; --k) {
         Level<T>& l = lv[k];
-        const int64_t n = pad(l.g.n), nL = pad(l.g.n * D), nr = pad(2 * (int64_t)l.g.N[1] * l.g.N[2]);
+        const int64_t n = pad(l.g.n), nL = pad(l.g.n * D), nr = pad((int64_t)l.g.N[1] * l.g.N[2]);
         if (pass == 1) {
           l.L = arena + o;
           l.r = l.L + nL;
@@ -359,7 +359,7 @@ struct MG {
     l0.ownz = !z0;
     l0.r = dalloc<T>(l0.g.n);
     l0.e = dalloc<T>(l0.g.n);
-    l0.lrow = dalloc<uint8_t>(2 * (int64_t)l0.g.N[1] * l0.g.N[2]);
+    l0.lrow = dalloc<uint8_t>((int64_t)l0.g.N[1] * l0.g.N[2]);
     {
       const char* e = std::getenv("WL_LROWS");
       use_lrows = !e || std::atoi(e) != 0;
@@ -477,44 +477,77 @@ struct MG {
     KCK();
   }
 
-  // Uniform-row flags of level l from its current L (WL_LROWS=0 disables the fast rows).
+  // What the solver keeps of the levels' L besides it, from the current L: the uniform-row flags (of
+  // every level, or those of one; WL_LROWS=0: none), with all also the fast tail's image, and the lean
+  // levels' 1/D and segment flags
   bool use_lrows = true;
   int lrow_epoch0 = 0;  // counts the rebuilds of the finest level's flags
-  void build_lrows(int l) {
+  void build_tables(bool all) {
+    Tables<T> d;
+    std::memset(&d, 0, sizeof d);
+    int nblk = 0;
+    bool in_lds = false;
+    const int Lt = tail_start(&in_lds);
+    const bool image = all && Lt >= 1 && in_lds && tail_fast(Lt);
+    TailFast<T> td;
+    if (image) {
+      td = tail_desc(Lt);
+      if (!tail_img) tail_img = dalloc<T>(td.nimg);
+    }
+    auto flush = [&] {
+      if (nblk) {
+        hipLaunchKernelGGL(k_level_tables<T>, dim3((unsigned)nblk), dim3(256), 0, st, d);
+        KCK();
+      }
+      d.n = nblk = 0;
+    };
+    for (int l = 0; l < (int)lv.size(); ++l) {
+      Level<T>& p = lv[l];
+      if (!all && p.lrow_ok) continue;
+      if (l == 0) ++lrow_epoch0;
+      const bool img = image && l >= Lt;
+      p.lrow_ok = false;
+      if (p.iD) build_lean_tables(l);
+      if (!use_lrows && !img) continue;
+      if (d.n == TAB_MAX) flush();
+      TabLv<T>& q = d.lv[d.n++];
+      q.g = p.g;
+      q.L = p.L;
+      for (int i = 0; i < 3; ++i) q.c[i] = p.lc[i];
+      q.rows = p.lrow;
+      q.img = img ? tail_img + td.lv[l - Lt].oL : nullptr;
+      q.blk0 = nblk;
+      nblk += (int)(((int64_t)p.g.N[1] * p.g.N[2] + 3) / 4);
+      if (img) nblk += (int)((p.g.n + 255) / 256);
+      p.lrow_ok = use_lrows;
+    }
+    flush();
+  }
+  void build_lean_tables(int l) {
     Level<T>& p = lv[l];
-    const int64_t nr = (int64_t)p.g.N[1] * p.g.N[2];
-    p.lrow_ok = false;
-    if (l == 0) ++lrow_epoch0;
-    if (p.iD) {
-      Box b = box_inside(p.g);
-      hipLaunchKernelGGL(k_diag<T>, grid_of(b), kBlock, 0, st, p.g, b, (const T*)p.L, p.iD, 1);
-      KCK();
-    }
+    Box b = box_inside(p.g);
+    hipLaunchKernelGGL(k_diag<T>, grid_of(b), kBlock, 0, st, p.g, b, (const T*)p.L, p.iD, 1);
+    KCK();
     if (!use_lrows) return;
-    hipLaunchKernelGGL(k_lrow_bits<T>, dim3((unsigned)((nr + 3) / 4)), dim3(256), 0, st, p.g, (const T*)p.L,
-                       p.lc[0], p.lc[1], p.lc[2], p.lrow);
+    const int ns = lean_nseg(p.g);
+    const int64_t nk = (int64_t)p.g.N[1] * p.g.N[2] * ns;
+    hipLaunchKernelGGL(k_seg_bits<T>, dim3((unsigned)((nk + 3) / 4)), dim3(256), 0, st, p.g, (const T*)p.L, p.lc[0],
+                       p.lc[1], p.lc[2], ns, p.lseg);
     KCK();
-    hipLaunchKernelGGL(k_lrow_flags, dim3((unsigned)((nr + 255) / 256)), dim3(256), 0, st, p.g,
-                       (const uint8_t*)p.lrow, p.lrow + nr);
+    hipLaunchKernelGGL(k_seg_uniform, dim3((unsigned)((nk + 255) / 256)), dim3(256), 0, st, p.g, ns,
+                       (const uint8_t*)p.lseg, p.lseg + nk);
     KCK();
-    if (p.iD) {
-      const int ns = lean_nseg(p.g);
-      const int64_t nk = nr * ns;
-      hipLaunchKernelGGL(k_seg_bits<T>, dim3((unsigned)((nk + 3) / 4)), dim3(256), 0, st, p.g, (const T*)p.L, p.lc[0],
-                         p.lc[1], p.lc[2], ns, p.lseg);
-      KCK();
-      hipLaunchKernelGGL(k_seg_uniform, dim3((unsigned)((nk + 255) / 256)), dim3(256), 0, st, p.g, ns,
-                         (const uint8_t*)p.lseg, p.lseg + nk);
-      KCK();
-      hipLaunchKernelGGL(k_seg_fast, dim3((unsigned)((nk + 255) / 256)), dim3(256), 0, st, p.g, ns,
-                         (const uint8_t*)p.lseg + nk, p.lseg + 2 * nk);
-      KCK();
-    }
-    p.lrow_ok = true;
+    hipLaunchKernelGGL(k_seg_fast, dim3((unsigned)((nk + 255) / 256)), dim3(256), 0, st, p.g, ns,
+                       (const uint8_t*)p.lseg + nk, p.lseg + 2 * nk);
+    KCK();
   }
   void ensure_lrows() {
-    for (size_t l = 0; l < lv.size(); ++l)
-      if (!lv[l].lrow_ok) build_lrows((int)l);
+    if (!use_lrows) return;
+    for (auto& p : lv)
+      if (!p.lrow_ok) {
+        build_tables(false);
+        return;
+      }
   }
   // the buffer Jacobi! reads ϵ from on level l
   T* jac(int l) const { return lv[l].ej ? lv[l].ej : lv[l].e; }
@@ -670,25 +703,36 @@ struct MG {
   double gs_bytes(int l) const { return (double)sizeof(T) * 1.5 * ncells_inside(lv[l].g); }
   LRows<T> lr(int l) const {
     const Level<T>& p = lv[l];
-    return LRows<T>{p.L, p.lrow_ok ? p.lrow + (int64_t)p.g.N[1] * p.g.N[2] : nullptr, {p.lc[0], p.lc[1], p.lc[2]}};
+    return LRows<T>{p.L, p.lrow_ok ? p.lrow : nullptr, {p.lc[0], p.lc[1], p.lc[2]}};
   }
   // update!(ml): coarse L by restrictL!, then BC!(L,0) (src/MultiLevelPoisson.jl:42-48,79-86);
   // then the uniform-row flags of every level
   void update() {
-    const double zero[3] = {0, 0, 0};
-    for (size_t l = 1; l < lv.size(); ++l) {
+    size_t l = 1;
+    for (; l < lv.size() && lv[l].g.n > chain_cells; ++l) {
       const Level<T>& f = lv[l - 1];
       Level<T>& c = lv[l];
-      Box b = box_inside(c.g);
-      if (!box_empty(b)) {
-        hipLaunchKernelGGL(k_restrictL<T>, grid_of(b), kBlock, 0, st, f.g, c.g, b, f.cmask, f.L, c.L);
-        KCK();
-      }
-      bc_vec(c.g, c.L, zero, 0);
+      Box b = box_all(c.g);
+      hipLaunchKernelGGL(k_restrictL<T>, grid_of(b), kBlock, 0, st, f.g, c.g, b, f.cmask, perdir, (const T*)f.L, c.L);
+      KCK();
     }
-    for (size_t l = 0; l < lv.size(); ++l) build_lrows((int)l);
-    build_tail_image();
+    while (l < lv.size()) {
+      ChainL<T> d;
+      std::memset(&d, 0, sizeof d);
+      d.perdir = perdir;
+      for (size_t k = l - 1; k < lv.size() && d.n < TAB_MAX; ++k, ++d.n) {
+        d.g[d.n] = lv[k].g;
+        d.L[d.n] = lv[k].L;
+        d.cm[d.n] = lv[k].cmask;
+      }
+      hipLaunchKernelGGL(k_restrictL_chain<T>, dim3(1), dim3(1024), 0, st, d);
+      KCK();
+      l += d.n - 1;
+    }
+    build_tables(true);
   }
+  // levels of at most so many cells are restricted by one block (four passes of its threads for the first)
+  static constexpr int64_t chain_cells = 4096;
 
   // mode 0: Σ into dsc[slot]; 1: also the mean and its flag (tsc[0..1]); 2 and 3 (slot 1): then the
   // solver's init or ω control on the device state, as k_mg_init / k_mg_control would
@@ -938,7 +982,7 @@ struct MG {
       if (tail_bytes((int)l) <= TAIL_LDS_BYTES) { *in_lds = true; return (int)l; }
     return -1;
   }
-  // the fast tail's image of L, D and 1/D (k_tail_image), formed with L in update()
+  // the fast tail's image of L, D and 1/D (k_level_tables), formed with L in update()
   T* tail_img = nullptr;
   TailFast<T> tail_desc(int Lt) const {
     TailFast<T> d;
@@ -975,19 +1019,6 @@ struct MG {
   static size_t tail_desc_lds(const TailFast<T>& d) {
     const TailLv& q = d.lv[d.n - 1];
     return (size_t)(q.oE + q.n) * sizeof(T);
-  }
-  void build_tail_image() {
-    bool in_lds = false;
-    const int Lt = tail_start(&in_lds);
-    if (Lt < 1 || !in_lds || !tail_fast(Lt)) return;
-    TailFast<T> d = tail_desc(Lt);
-    if (!tail_img) tail_img = dalloc<T>(d.nimg);
-    for (int k = 0; k < d.n; ++k) {
-      const Level<T>& q = lv[Lt + k];
-      hipLaunchKernelGGL(k_tail_image<T>, dim3((unsigned)((q.g.n + 255) / 256)), dim3(256), 0, st, q.g,
-                         (const T*)q.L, tail_img + d.lv[k].oL);
-      KCK();
-    }
   }
   bool exact_coarsest = false;  // set by the mixed-precision loop around its V-cycles
   bool coarse_pcg = false;      // WL_COARSE_PCG=1: that coarsest level by FP64 pcg! instead of GS-RB
@@ -1755,21 +1786,17 @@ struct FlowT : FlowBase {
   void measure(const wl_body* b, int nb, double t, double eps) override {
     (void)t;
     DBodies bs = to_dbodies(b, nb);
-    const int64_t n = g.n;
-    fill(V, n * D, T(0));
-    fill(mu0, n * D, T(1));
-    fill(mu1, n * D * D, T(0));
     const T d2 = (T)(2 + eps) * (T)(2 + eps);
-    Box bi = box_inside(g);
-    hipLaunchKernelGGL(k_measure_sdf<T>, grid_of(bi), kBlock, 0, st, g, bi, bs, sigma, d2);
+    const int64_t nr = (int64_t)g.N[1] * g.N[2];
+    hipLaunchKernelGGL(k_fill<uint8_t>, dim3((unsigned)((2 * nr + 255) / 256)), dim3(256), 0, st, rows, 2 * nr,
+                       (uint8_t)0);
     KCK();
-    hipLaunchKernelGGL(k_measure_fill<T>, grid_of(bi), kBlock, 0, st, g, bi, bs, (const T*)sigma, V, mu0, mu1, d2,
-                       (T)eps);
+    Box ba = box_all(g);
+    hipLaunchKernelGGL(k_measure<T>, grid_of(ba), kBlock, 0, st, g, ba, bs, sigma, V, mu0, mu1, d2, (T)eps,
+                       desc.perdir_mask, rows);
     KCK();
-    const double zero[3] = {0, 0, 0};
-    mg.bc_vec(g, mu0, zero, 0);
-    mg.bc_vec(g, V, zero, desc.exit_bc);
-    mu1_dirty = true;
+    mu1_dirty = false;
+    crows_ok = false;
     mg.lv[0].lrow_ok = false;
     sync();
   }
@@ -1782,15 +1809,13 @@ struct FlowT : FlowBase {
   void conv_rows() {
     const int64_t nr = (int64_t)g.N[1] * g.N[2];
     const LRows<T> m0 = mg.lr(0);
-    int* cnt = rlist + nr;
     hipLaunchKernelGGL(k_conv_rows, dim3((unsigned)((nr + 255) / 256)), dim3(256), 0, st, g, (const uint8_t*)rows,
                        (const uint8_t*)vrows(), m0.rows, crows());
     KCK();
-    hipLaunchKernelGGL(k_row_list, dim3(1), dim3(1024), 0, st, g, (const uint8_t*)crows(), rlist, cnt);
+    host_unset(B, HOST_ROWS);
+    hipLaunchKernelGGL(k_row_list, dim3(1), dim3(1024), 0, st, g, (const uint8_t*)crows(), rlist, B.host);
     KCK();
-    HIPCK(hipMemcpyAsync(B.hsc, cnt, sizeof(int), hipMemcpyDeviceToHost, st));
-    HIPCK(hipStreamSynchronize(st));
-    std::memcpy(&nlist, B.hsc, sizeof(int));
+    nlist = (int)host_wait(B, HOST_ROWS, st);
     crows_ok = true;
     crows_epoch = mg.lrow_epoch0;
   }
