@@ -117,6 +117,23 @@ __device__ __forceinline__ double block_sum(double v) {
   __syncthreads();
   return v;
 }
+// n sums at once, each in block_sum's order; the results are valid in thread 0
+template <int N>
+__device__ __forceinline__ void block_sum_n(double* v) {
+  __shared__ double sh[N][16];
+  const int t = threadIdx.x + blockDim.x * threadIdx.y;
+  const int nw = (blockDim.x * blockDim.y + 63) >> 6;
+#pragma unroll
+  for (int q = 0; q < N; ++q) v[q] = wave_sum(v[q]);
+  if ((t & 63) == 0)
+#pragma unroll
+    for (int q = 0; q < N; ++q) sh[q][t >> 6] = v[q];
+  __syncthreads();
+  if (t < 64)
+#pragma unroll
+    for (int q = 0; q < N; ++q) v[q] = wave_sum(t < nw ? sh[q][t] : 0.0);
+  __syncthreads();
+}
 template <class T>
 __device__ __forceinline__ T block_max(T v, T ident) {
   __shared__ T shm[16];
