@@ -1725,6 +1725,7 @@ struct FlowT : FlowBase {
       }
     }
     alloc_bufs(B, 3 * nblocks(box_all(g)) + 16, sizeof(T));
+    if (d.exit_bc && exit_cells(g) > EXIT_ONE) exit_q = dalloc<T>(3 * exit_cells(g));
     mg.st = st;
     mg.B = &B;
     mg.P = &prof;
@@ -1747,7 +1748,7 @@ struct FlowT : FlowBase {
   }
   ~FlowT() override {
     (void)hipStreamSynchronize(st);
-    dfree(u); dfree(u0); dfree(u1); dfree(rlist); dfree(f); dfree(V); dfree(mu0); dfree(mu1); dfree(p); dfree(sigma); dfree(xw);
+    dfree(u); dfree(u0); dfree(u1); dfree(rlist); dfree(f); dfree(V); dfree(mu0); dfree(mu1); dfree(p); dfree(sigma); dfree(xw); dfree(exit_q);
     dfree(rows);
     dfree(mpart); dfree(fn_ubc); dfree(fn_acc[0]); dfree(fn_acc[1]);
     free_bufs(B);
@@ -2054,9 +2055,19 @@ struct FlowT : FlowBase {
     if (pred && desc.exit_bc) exit_bc(u0, dt);  // src/Flow.jl:195, predictor only
   }
   // exitBC!(u, src, Δt) (src/core.jl:226-233)
+  T* exit_q = nullptr;  // k_exit_gather's planes (exitBC, more than EXIT_ONE cells)
   void exit_bc(const T* src, T dt) {
     ProfScope ps(&prof, st, "exit_bc", 0, 0.0);
-    hipLaunchKernelGGL(k_exit_bc<T>, dim3(1), dim3(1024), 0, st, g, u, src, dt);
+    const dim3 gd((unsigned)((exit_cells(g) + 255) / 256));
+    if (exit_q) {
+      hipLaunchKernelGGL(k_exit_gather<T>, gd, dim3(256), 0, st, g, (const T*)u, src, exit_q);
+      KCK();
+      hipLaunchKernelGGL((k_exit_bc<T, true>), dim3(1), dim3(1024), 0, st, g, u, src, dt, exit_q);
+      KCK();
+      hipLaunchKernelGGL(k_exit_scatter<T>, gd, dim3(256), 0, st, g, u, (const T*)exit_q);
+    } else {
+      hipLaunchKernelGGL((k_exit_bc<T, false>), dim3(1), dim3(1024), 0, st, g, u, src, dt, (T*)nullptr);
+    }
     KCK();
   }
 
