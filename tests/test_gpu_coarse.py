@@ -92,6 +92,29 @@ def test_lean_equals_plain(wl, how, T, monkeypatch):
         assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("T", [np.float32, np.float64])
+@pytest.mark.parametrize("n", [(72, 40), (64, 33), (32, 24, 16), (128, 40, 40)], ids=lambda v: "x".join(map(str, v)))
+def test_launches_ahead_of_the_read(wl, n, T, monkeypatch):
+    """The launches issued before the host has read Σr² (guessed from the last solve's V-cycles) against
+    a run that issues none (a profiled flow), while the tolerance and the limit make the guess wrong
+    both ways: the same V-cycles, u and p."""
+    print("case: launches ahead", n, T.__name__, flush=True)
+    monkeypatch.setenv("WL_LEAN", "2" if n[0] == 128 else "1")
+    D, R, got = len(n), min(n) / 5, []
+    for profiled in (True, False):
+        sim = wl.Simulation(n, (1,) + (0,) * (D - 1), 2 * R, ν=R / 50, body=wl.Sphere(tuple(v / 2 for v in n), R), T=T)
+        sim.flow.profile(profiled)
+        out = []
+        for kw in ({}, dict(tol=1e-7), dict(tol=1e-7), dict(itmx=1), dict(tol=1e-7, itmx=2), dict(tol=1e-1), {}):
+            sim.pois.set_solver(**kw)
+            wl.sim_step(sim, remeasure=False)
+            out += [sim.flow.get("u"), sim.flow.get("p")]
+        got.append((list(sim.pois.n), out))
+    assert got[0][0] == got[1][0] and len(set(got[0][0])) > 2
+    for a, b in zip(got[0][1], got[1][1]):
+        assert np.array_equal(a, b)
+
+
 def bc_fill(a, perdir, value=0):
     """BC!(a, value) (src/core.jl:200-219) of a vector field without exit, in the reference's loops."""
     D = a.ndim - 1

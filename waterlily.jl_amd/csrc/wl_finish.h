@@ -43,12 +43,26 @@ __device__ __forceinline__ void host_post(double* __restrict__ host, int slot, d
   __hip_atomic_store((unsigned long long*)host + slot, b, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// What a control decides besides ω: whether another iteration follows (the host's own tests, with its
+// tolerance; last: the iteration limit is reached).  A launch that is issued before the host has read
+// Σr² carries a Gate and ends at once where the decision was the other one.
+struct Next {
+  int* go;
+  double tol;
+  int last;
+};
+struct Gate {
+  const int* go;  // nullptr: no condition
+  int want;
+  __device__ __forceinline__ bool closed() const { return go != nullptr && *go != want; }
+};
 enum FinMode { FIN_SUM = 0, FIN_MEAN = 1, FIN_INIT = 2, FIN_CONTROL = 3 };
 // what follows from the sum s: FIN_MEAN (residual!): the mean in T and whether it is removed (st[0..1]);
 // FIN_INIT, FIN_CONTROL: the solver's state, the host then told of a control's Σr²
 template <class T>
 __device__ __forceinline__ void fin_apply(int mode, double s, double* __restrict__ outd, T* __restrict__ st, double ninside,
-                                          double* __restrict__ dsc, double* __restrict__ host) {
+                                          double* __restrict__ dsc, double* __restrict__ host,
+                                          Next next = Next{nullptr, 0, 0}) {
   outd[0] = s;
   if (mode == FIN_MEAN) {
     const T sm = (T)s / (T)ninside;
@@ -58,6 +72,7 @@ __device__ __forceinline__ void fin_apply(int mode, double s, double* __restrict
   if (mode == FIN_INIT) mg_init_state<T>(s, st);
   if (mode == FIN_CONTROL) {
     mg_control_state<T>(s, dsc, st);
+    if (next.go) *next.go = !((double)(T)s < next.tol) && isfinite((T)s) && !next.last;
     if (host) {
       host[HOST_R2_OLD] = dsc[6];
       host_post(host, HOST_R2, s);

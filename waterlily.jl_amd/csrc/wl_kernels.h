@@ -797,7 +797,8 @@ __device__ __forceinline__ void k_bc_body(const Geo& g, T* __restrict__ a, int n
 }
 template <class T>
 __global__ void __launch_bounds__(256) k_bc(Geo g, T* __restrict__ a, int ncomp_vec, double U0, double U1,
-                                            double U2, int saveexit, int perdir) {
+                                            double U2, int saveexit, int perdir, Gate gate = Gate{nullptr, 0}) {
+  if (gate.closed()) return;
   k_bc_body<T>(g, a, ncomp_vec, U0, U1, U2, saveexit, perdir, (int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z);
 }
 
@@ -1927,7 +1928,8 @@ template <class T, int D>
 __global__ void __launch_bounds__(256) k_inc_restrict2(Geo gf, Geo gc, ZT t, LRows<T> Lf, T* __restrict__ rf,
                                                        T* __restrict__ xf, const T* __restrict__ ef,
                                                        LRows<T> Lc, T* __restrict__ rc, T* __restrict__ xc,
-                                                       T* __restrict__ ec) {
+                                                       T* __restrict__ ec, Gate gate) {
+  if (gate.closed()) return;
   int cx, cy, z0, z1;
   zt_cell(t, cx, cy, z0, z1);  // threadIdx.x (0..63) is remapped below: the tile is 32 x wide
   const int lane = threadIdx.x, half = lane >> 5;
@@ -2514,7 +2516,8 @@ __device__ __forceinline__ void k_correct_body(const Geo& g, const ZT& t, T* __r
 }
 template <class T>
 __global__ void __launch_bounds__(256) k_correct(Geo g, ZT t, T* __restrict__ u, LRows<T> LR,
-                                                 const T* __restrict__ x, T* __restrict__ p, T dt) {
+                                                 const T* __restrict__ x, T* __restrict__ p, T dt, Gate gate) {
+  if (gate.closed()) return;
   k_correct_body<T>(g, t, u, LR, x, p, dt, xcd_tile_id());
 }
 
@@ -2580,13 +2583,14 @@ template <class T>
 __global__ void __launch_bounds__(1024) k_finish_sum(const double* __restrict__ partial, int64_t np,
                                                      double* __restrict__ outd, T* __restrict__ outT, int mode,
                                                      double ninside, double* __restrict__ dsc = nullptr,
-                                                     double* __restrict__ host = nullptr) {
+                                                     double* __restrict__ host = nullptr,
+                                                     Next next = Next{nullptr, 0, 0}) {
   // each thread's partials in index order; the loads run ahead of the dependent adds
   double acc = 0;
 #pragma unroll 8
   for (int64_t q = threadIdx.x; q < np; q += blockDim.x) acc += partial[q];
   const double s = block_sum(acc);
-  if (threadIdx.x == 0) fin_apply<T>(mode, s, outd, outT, ninside, dsc, host);
+  if (threadIdx.x == 0) fin_apply<T>(mode, s, outd, outT, ninside, dsc, host, next);
 }
 template <class T>
 __global__ void __launch_bounds__(1024) k_finish_max(const T* __restrict__ partial, int64_t np, double* __restrict__ host) {

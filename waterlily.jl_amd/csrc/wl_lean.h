@@ -296,7 +296,8 @@ __device__ __forceinline__ void lean_mode(const Geo& g, bool fast, int z, F&& f)
 template <class T, bool CE>
 __global__ void __launch_bounds__(256) k_lean_restrict(Geo gf, Geo gc, ZT t, LeanL<T> A, const T* __restrict__ r,
                                                        LRows<T> Lc, T* __restrict__ rc, T* __restrict__ xc,
-                                                       T* __restrict__ ec) {
+                                                       T* __restrict__ ec, Gate gate) {
+  if (gate.closed()) return;
   int cx, cy, z0, z1;
   zt_cell_id(t, lean_tile(t), cx, cy, z0, z1);  // the tile is 32 coarse cells wide
   const int lane = threadIdx.x, half = lane >> 5;

@@ -8,6 +8,7 @@
 #include <cstring>
 #include <cmath>
 #include <chrono>
+#include <functional>
 #include <string>
 #include <vector>
 #include <memory>
@@ -243,6 +244,7 @@ struct Bufs {  // reduction scratch shared by a handle
   void* tsc = nullptr;     // device T scalars
   double* hsc = nullptr;   // pinned host doubles
   unsigned* cnt = nullptr; // blocks of the running launch that have ended (fin_last)
+  int* go = nullptr;       // whether a further solver iteration follows (Next, Gate)
   double* host = nullptr;  // coherent pinned host doubles (HostSlot): what the host waits for
 };
 
@@ -451,7 +453,7 @@ struct MG {
     }
   }
 
-  void bc_vec(const Geo& g, T* a, const double* U, int saveexit) {
+  void bc_vec(const Geo& g, T* a, const double* U, int saveexit, Gate gate = Gate{nullptr, 0}) {
     ProfScope ps(P, st, "bc", 0, 0.0);
     int maxplane = 0;
     for (int d = 0; d < g.D; ++d) {
@@ -460,7 +462,8 @@ struct MG {
       maxplane = std::max(maxplane, p);
     }
     dim3 gd((maxplane + 255) / 256, g.D, 2 * g.D + 1);
-    hipLaunchKernelGGL(k_bc<T>, gd, dim3(256), 0, st, g, a, 1, U[0], U[1], g.D > 2 ? U[2] : 0.0, saveexit, perdir);
+    hipLaunchKernelGGL(k_bc<T>, gd, dim3(256), 0, st, g, a, 1, U[0], U[1], g.D > 2 ? U[2] : 0.0, saveexit, perdir,
+                       gate);
     KCK();
   }
   template <class U>
@@ -606,7 +609,7 @@ struct MG {
     return t;
   }
   T* lean_eps(int l) const { return l == 0 ? lv[0].e : lv[l].se; }  // lv[0].e: between split_begin and _end
-  void restrict_lean(int l) {
+  void restrict_lean(int l, Gate gate) {
     Level<T>& f = lv[l];
     Level<T>& c = lv[l + 1];
     bool in_lds = false;
@@ -621,10 +624,10 @@ struct MG {
     bc.zc = 4;
     if (ce)
       hipLaunchKernelGGL((k_lean_restrict<T, true>), zt_grid(bc), kBlock, 0, st, f.g, c.g, bc, lean_args(l),
-                         (const T*)f.r, lr(l + 1), c.r, c.x, c.e);
+                         (const T*)f.r, lr(l + 1), c.r, c.x, c.e, gate);
     else
       hipLaunchKernelGGL((k_lean_restrict<T, false>), zt_grid(bc), kBlock, 0, st, f.g, c.g, bc, lean_args(l),
-                         (const T*)f.r, lr(l + 1), c.r, c.x, c.e);
+                         (const T*)f.r, lr(l + 1), c.r, c.x, c.e, gate);
     KCK();
   }
   // from level c into c − 1; fold: x + ω·ϵ of level c is formed at the cells read
@@ -739,7 +742,7 @@ struct MG {
   // the partials start at B->partial + poff
   double finish_sum(int64_t np, int slot, int mode = 0, double ninside = 1, int64_t poff = 0) {
     hipLaunchKernelGGL(k_finish_sum<T>, dim3(1), dim3(1024), 0, st, (const double*)B->partial + poff, np, B->dsc + slot,
-                       (T*)B->tsc, mode, ninside, B->dsc, B->host);
+                       (T*)B->tsc, mode, ninside, B->dsc, B->host, next);
     KCK();
     return 0;
   }
@@ -1120,7 +1123,8 @@ struct MG {
     bool in_lds = false;
     const int Lt = tail_start(&in_lds);
     const int down_end = Lt > 0 ? Lt : Lm;
-    for (int l = 0; l < down_end; ++l) restrict_level(l);  // down-leg: Jacobi! + restrict! + fill!
+    for (int l = ahead ? 1 : 0; l < down_end; ++l) restrict_level(l);  // down-leg: Jacobi! + restrict! + fill!
+    ahead = false;
     if (Lt > 0) launch_tail(Lt, in_lds, w);  // levels Lt..Lm, through smooth!(Lt)
     bool done = Lt > 0;  // the coarse level's smooth! and increment! are done
     for (int c = Lt > 0 ? Lt : Lm; c >= 1; --c) {  // up-leg: smooth!(coarse), prolongate! + increment!(fine)
@@ -1192,9 +1196,13 @@ struct MG {
   }
   int64_t fin_blocks = 0;
   // Jacobi! (ω = 1) on level l, restrict! to l+1 and fill!(x, 0) there (src/MultiLevelPoisson.jl:92-94)
-  void restrict_level(int l) {
+  // (gate: only where restrict_gated says so)
+  bool restrict_gated(int l) const {
+    return lean(l) || (lv[l].cmask == (1 << lv[l].g.D) - 1 && use_pairs && perdir == 0);
+  }
+  void restrict_level(int l, Gate gate = Gate{nullptr, 0}) {
     if (lean(l)) {
-      restrict_lean(l);
+      restrict_lean(l, gate);
       return;
     }
     Level<T>& f = lv[l];
@@ -1212,13 +1220,12 @@ struct MG {
       const int64_t per = (int64_t)bc.nbx * bc.nby;
       const int nz = bc.b.hi[2] - bc.b.lo[2] + 1;
       bc.zc = (int)std::min<int64_t>(32, std::max<int64_t>(1, (int64_t)nz * per / tgt_rp()));
-    if (std::getenv("R_ZC")) bc.zc = std::atoi(std::getenv("R_ZC"));
       if (f.g.D == 3)
         hipLaunchKernelGGL((k_inc_restrict2<T, 3>), zt_grid(bc), kBlock, 0, st, f.g, c.g, bc, lr(l), f.r, f.x,
-                           (const T*)fe, lr(l + 1), c.r, c.x, c.e);
+                           (const T*)fe, lr(l + 1), c.r, c.x, c.e, gate);
       else
         hipLaunchKernelGGL((k_inc_restrict2<T, 2>), zt_grid(bc), kBlock, 0, st, f.g, c.g, bc, lr(l), f.r, f.x,
-                           (const T*)fe, lr(l + 1), c.r, c.x, c.e);
+                           (const T*)fe, lr(l + 1), c.r, c.x, c.e, gate);
     } else if (f.cmask == full) {
       // fine x,y tile ranges, coarse z planes (the fine inside extents are even here)
       Box b = box_inside(f.g);
@@ -1424,7 +1431,17 @@ struct MG {
   // solver!(ml) loop (src/MultiLevelPoisson.jl:108-127) after residual!: returns V-cycle count.
   // The host reads Σr² back once per iteration for the stop test, as the reference does.
   // init_done: mean_l2(true) has already set the start state.
-  int mg_loop(double tol, int itmx, std::vector<double>* hist, bool init_done = false) {
+  //
+  // Between an iteration's last launch and the host's next one lie its read of Σr² and a launch, some 8
+  // us.  So the next launches are issued ahead of that read, gated on the iteration's own decision:
+  // where the last solve of this kind (`like`, in its V-cycles) went on at this count, the next
+  // V-cycle's first pass; where it ended, what follows the solve (`after`).  A wrong guess costs launches
+  // that do nothing.  *after_done: `after` ran.  Step, us: 64x64 137 -> 123, 192x128 159 -> 146,
+  // 1024x512 258 -> 244, 96x64x64 325 -> 308, 208x112x80 644 -> 630.
+  bool ahead = false;  // the next V-cycle's first pass has been issued
+  Next next{nullptr, 0, 0};
+  int mg_loop(double tol, int itmx, std::vector<double>* hist, bool init_done = false, int like = 0,
+              const std::function<void(Gate)>& after = nullptr, bool* after_done = nullptr) {
     if (!init_done) {
       hipLaunchKernelGGL(k_mg_init<T>, dim3(1), dim3(64), 0, st, (const double*)B->dsc, (T*)B->tsc);
       KCK();
@@ -1433,20 +1450,35 @@ struct MG {
     if (itmx <= 0) {
       if (hist) hist->push_back((double)(T)read_dsc(1));
     }
+    const bool issue = !use_graphs && !(P && P->on);
+    bool in_lds = false;
+    const bool down0 = tail_start(&in_lds) != 0;  // a V-cycle starts with a pass of the finest level
+    ahead = false;
     while (n < itmx) {
       host_unset(*B, HOST_R2);
+      next = issue ? Next{B->go, tol, n + 1 >= itmx} : Next{nullptr, 0, 0};
       run_iteration(n == 0);
+      next = Next{nullptr, 0, 0};
+      bool first_pass = false, followed = false;
+      if (issue && n + 1 < like) {
+        first_pass = down0 && restrict_gated(0) && (ej_written || lean_on);
+        if (first_pass) restrict_level(0, Gate{B->go, 1});
+      } else if (issue && after) {
+        after(Gate{B->go, 0});
+        followed = true;
+      }
       const T rnew = (T)host_wait(*B, HOST_R2, st);
       if (hist) {
         if (n == 0) hist->push_back(B->host[HOST_R2_OLD]);
         hist->push_back((double)rnew);
       }
       n++;
-      if ((double)rnew < tol) break;
-      if (!std::isfinite(rnew)) {  // NaN/Inf reached Σr²: further V-cycles cannot recover it
-        nan_seen = true;
+      if (!std::isfinite(rnew)) nan_seen = true;  // NaN/Inf reached Σr²: further V-cycles cannot recover it
+      if ((double)rnew < tol || !std::isfinite(rnew) || n >= itmx) {
+        if (after_done) *after_done = followed;
         break;
       }
+      ahead = first_pass;
     }
     if (fin_r && lv[0].r != r_home) std::swap(lv[0].r, fin_r);  // (its values are not read again)
     perbc(lv[0].g, lv[0].x);
@@ -1615,6 +1647,7 @@ static void alloc_bufs(Bufs& B, int64_t np, size_t tsize) {
   (void)tsize;
   HIPCK(hipHostMalloc((void**)&B.hsc, 8 * sizeof(double), hipHostMallocDefault));
   B.cnt = dalloc<unsigned>(1);
+  B.go = dalloc<int>(1);
   HIPCK(hipHostMalloc((void**)&B.host, HOST_SLOTS * sizeof(double), hipHostMallocCoherent));
 }
 static void free_bufs(Bufs& B) {
@@ -1623,6 +1656,7 @@ static void free_bufs(Bufs& B) {
   dfree(B.tsc);
   if (B.hsc) (void)hipHostFree(B.hsc);
   dfree(B.cnt);
+  dfree(B.go);
   if (B.host) (void)hipHostFree(B.host);
 }
 
@@ -1874,11 +1908,11 @@ struct FlowT : FlowBase {
   }
   // BC! of u at time t: the uniform closed form, or the reference's sequential loops on the
   // function field (src/core.jl:200-219)
-  void apply_bc_u(double t) {
+  void apply_bc_u(double t, Gate gate = Gate{nullptr, 0}) {  // (gate: the closed form only)
     if (!use_ubc) {
       double Ub[3];
       Ut(t, Ub);
-      mg.bc_vec(g, u, Ub, desc.exit_bc);
+      mg.bc_vec(g, u, Ub, desc.exit_bc, gate);
       return;
     }
     ProfScope ps(&prof, st, "bc", 0, 0.0);
@@ -2116,7 +2150,7 @@ struct FlowT : FlowBase {
     ZT ba = make_zt_short(box_all(g), 8);
     {
     ProfScope ps(&prof, st, "correct", 0, (double)sizeof(T) * (2 * g.n + 2 * D * ncells_inside(g)));
-    hipLaunchKernelGGL(k_correct<T>, zt_grid(ba), kBlock, 0, st, g, ba, u, mg.lr(0), (const T*)xw, p, dt);
+    hipLaunchKernelGGL(k_correct<T>, zt_grid(ba), kBlock, 0, st, g, ba, u, mg.lr(0), (const T*)xw, p, dt, Gate{nullptr, 0});
     KCK();
     }
     apply_bc_u(t1);
@@ -2187,6 +2221,7 @@ struct FlowT : FlowBase {
   }
 
   // mom_project! (src/Flow.jl:223-232)
+  int last_nit[2] = {0, 0};  // V-cycles of the last predictor's and corrector's solve
   int project(T w, T dt_end, double t1) {
     if (mode == WL_SOLVER_MIXED) return project_mixed(w, dt_end, t1);
     const T dt = w * dt_end;
@@ -2220,15 +2255,23 @@ struct FlowT : FlowBase {
     // Σr²)
     mg.mean_l2(!use_net);
     if (use_net) warm_guess();
-    const int nit = mg.mg_loop(tol, itmx, &r2hist, !use_net);
+    const ZT ba = make_zt_short(box_all(g), 8);
+    auto correct = [&](Gate gate) {
+      ProfScope ps(&prof, st, "correct", 0, (double)sizeof(T) * (2 * g.n + 2 * D * ncells_inside(g)));
+      hipLaunchKernelGGL(k_correct<T>, zt_grid(ba), kBlock, 0, st, g, ba, u, mg.lr(0), (const T*)xw, p, dt, gate);
+      KCK();
+      apply_bc_u(t1, gate);
+    };
+    bool corrected = false;
+    int& like = last_nit[w == T(1) ? 0 : 1];
+    // (x's periodic ghosts and a network's record come between the solve and the correction; function
+    // boundary values are several launches)
+    std::function<void(Gate)> after;
+    if (!use_net && desc.perdir_mask == 0 && !use_ubc) after = correct;
+    const int nit = mg.mg_loop(tol, itmx, &r2hist, !use_net, like, after, &corrected);
+    like = nit;
     if (use_net && (net_flags & WL_WARM_RECORD)) net->record<T>(g, (const T*)xw, st);
-    ZT ba = make_zt_short(box_all(g), 8);
-    {
-    ProfScope ps(&prof, st, "correct", 0, (double)sizeof(T) * (2 * g.n + 2 * D * ncells_inside(g)));
-    hipLaunchKernelGGL(k_correct<T>, zt_grid(ba), kBlock, 0, st, g, ba, u, mg.lr(0), (const T*)xw, p, dt);
-    KCK();
-    }
-    apply_bc_u(t1);
+    if (!corrected) correct(Gate{nullptr, 0});
     return nit;
   }
 
