@@ -199,6 +199,17 @@ __global__ void __launch_bounds__(256) kb_prolong(const ALev<T>* __restrict__ A,
   else
     k_prolong_inc_body<T, false>(a.g, a.gc, a.t, a.cm, a.perdir, a.L, a.r, a.x, a.e, a.xc, a.wp, b.lid);
 }
+// The up-leg of one level of the simulations that take it in one launch (k_up), as each does when it
+// is stepped alone: one launch for a prolongation and four half sweeps.  64 uneven 2D simulations,
+// 2.2 M cells: two levels below the finest 24 + 27 us per V-cycle in ten launches, now two.
+template <class T, int D>
+__global__ void __launch_bounds__((UpTile<D, false>::THREADS)) kb_up(const UpArgs<T>* __restrict__ A,
+                                                                     const BBlk* __restrict__ blk,
+                                                                     const int* __restrict__ act) {
+  const BBlk b = blk[blockIdx.x];
+  if (!act[b.sim]) return;
+  k_up_body<T, D, false>(A[b.sim], b.lid, b.pidx);
+}
 // the coarse tail of each simulation: one workgroup per simulation (k_mg_tail_fast, or k_mg_tail_lds
 // where its first level has more x pairs than threads)
 template <class T>

@@ -844,7 +844,7 @@ __device__ __forceinline__ PairCoef<T, D> pair_coef(const LC<T>& a, const LC<T>&
   return c;
 }
 template <class T, int D, bool FIN>
-__device__ __forceinline__ void k_up_body(const UpArgs<T>& a, int bid, int nb, int pidx) {
+__device__ __forceinline__ void k_up_body(const UpArgs<T>& a, int lid, int pidx) {
   using U = UpTile<D, FIN>;
   constexpr int H = U::H, NI = U::NI, SX = U::SX, SXY = U::SX * U::SY;
   extern __shared__ __align__(16) unsigned char up_smem[];
@@ -852,7 +852,6 @@ __device__ __forceinline__ void k_up_body(const UpArgs<T>& a, int bid, int nb, i
   const T w = *a.w;
   const int tid = threadIdx.x;
   const int N[3] = {a.gf.N[0], a.gf.N[1], a.gf.N[2]};
-  const int lid = xcd_tile_of(bid, nb);
   const int tx = lid % a.ntx, t1 = lid / a.ntx, ty = t1 % a.nty, tz = t1 / a.nty;
   // the region's first cell
   const int bx = 1 + tx * U::OX - H, by = 1 + ty * U::OY - H, bz = D == 3 ? 1 + tz * U::OZ - H : 0;
@@ -986,7 +985,7 @@ __device__ __forceinline__ void k_up_body(const UpArgs<T>& a, int bid, int nb, i
 }
 template <class T, int D, bool FIN>
 __global__ void __launch_bounds__((UpTile<D, FIN>::THREADS)) k_up(UpArgs<T> a) {
-  k_up_body<T, D, FIN>(a, (int)blockIdx.x, (int)gridDim.x, (int)blockIdx.x);
+  k_up_body<T, D, FIN>(a, xcd_tile_id(), (int)blockIdx.x);
 }
 
 }  // namespace wl

@@ -2519,6 +2519,20 @@ struct BatchT : BatchBase {
     return a;
   }
 
+  // Levels below the finest that member s runs by k_up, as alone (MG::up_ok); the level below them is
+  // the tail's or k_up's too
+  bool takes_up(int s, int l) const {
+    return l >= 1 && l < Lt[s] && F[s]->mg.up_ok(l) && (l + 1 >= Lt[s] || takes_up(s, l + 1));
+  }
+  std::vector<Launch> ups;  // per level
+  template <int DD>
+  static int64_t up_tiles(UpArgs<T>& a) {
+    using U = UpTile<DD, false>;
+    auto tiles = [](int n, int o) { return (n + o - 1) / o; };
+    a.ntx = tiles(a.gf.N[0] - 2, U::OX);
+    a.nty = tiles(a.gf.N[1] - 2, U::OY);
+    return (int64_t)a.ntx * a.nty * (DD == 3 ? tiles(a.gf.N[2] - 2, U::OZ) : 1);
+  }
   void build_static() {
     inc_full.resize(Cmax); inc_gen.resize(Cmax); gs.resize(Cmax + 1); incr.resize(Cmax + 1); pro.resize(Cmax + 1);
     for (int l = 0; l < Cmax; ++l) {  // down-leg l -> l+1
@@ -2549,10 +2563,24 @@ struct BatchT : BatchBase {
     }
     for (int l = 0; l <= Cmax; ++l) {
       std::vector<ALev<T>> ags, agi, agp;
-      std::vector<BBlk> bgs, bgi, bgp;
+      std::vector<UpArgs<T>> aup;
+      std::vector<BBlk> bgs, bgi, bgp, bup;
       for (int s = 0; s < ns; ++s) {
-        const bool smooth = l == 0 || l < Lt[s];  // levels smoothed outside the tail
-        const bool prol = l < Lt[s];              // prolongation into level l from l+1
+        const bool up = takes_up(s, l);
+        const bool smooth = l == 0 || (l < Lt[s] && !up);  // levels smoothed outside the tail and k_up
+        const bool prol = l < Lt[s] && !up;                // prolongation into level l from l+1
+        {
+          UpArgs<T> a;
+          std::memset(&a, 0, sizeof a);
+          if (up) {
+            MG<T>& mg = F[s]->mg;
+            const Level<T>& f = mg.lv[l];
+            const Level<T>& c = mg.lv[l + 1];
+            a = UpArgs<T>{f.g, c.g, f.cmask, 0, mg.lr(l), f.r, f.x, c.x, (const T*)F[s]->B.tsc + 3, nullptr, nullptr, nullptr, 0, 0};
+            add_blocks(bup, s, D == 3 ? up_tiles<3>(a) : up_tiles<2>(a));
+          }
+          aup.push_back(a);
+        }
         const Geo& g = F[s]->mg.lv[l < (int)F[s]->mg.lv.size() ? l : 0].g;
         if (smooth) {
           const ZT th = make_zt(box_half(g), F[s]->mg.tgt_gs_at(l));
@@ -2567,7 +2595,8 @@ struct BatchT : BatchBase {
         if (prol) {
           const ZT tp = make_zt(box_inside(g), F[s]->mg.tgt_rp());
           agp.push_back(lev_args(F[s], l, tp));
-          agp.back().cinc = l + 1 < Lt[s] ? 1 : 0;  // level l+1 smoothed by launches: fold its increment!
+          // level l+1 smoothed by launches: fold its increment!
+          agp.back().cinc = l + 1 < Lt[s] && !takes_up(s, l + 1) ? 1 : 0;
           add_blocks(bgp, s, zt_blocks(tp));
         } else {
           agp.push_back(ALev<T>{});
@@ -2576,6 +2605,7 @@ struct BatchT : BatchBase {
       gs[l] = make_launch(ags, bgs);
       incr[l] = make_launch(agi, bgi);
       pro[l] = make_launch(agp, bgp);
+      ups.push_back(make_launch(aup, bup));
     }
     incr0 = incr[0];
     {
@@ -2822,6 +2852,16 @@ struct BatchT : BatchBase {
       const Launch& P = pro[c - 1];
       if (P.nblk) {
         hipLaunchKernelGGL(kb_prolong<T>, dim3(P.nblk), kBlock, 0, st, (const ALev<T>*)P.args, P.blk, (const int*)act);
+        KCK();
+      }
+      const Launch& u = ups[c - 1];
+      if (u.nblk) {
+        if (D == 3)
+          hipLaunchKernelGGL((kb_up<T, 3>), dim3(u.nblk), dim3(UpTile<3, false>::THREADS), (up_lds<T, 3, false>()), st,
+                             (const UpArgs<T>*)u.args, u.blk, (const int*)act);
+        else
+          hipLaunchKernelGGL((kb_up<T, 2>), dim3(u.nblk), dim3(UpTile<2, false>::THREADS), (up_lds<T, 2, false>()), st,
+                             (const UpArgs<T>*)u.args, u.blk, (const int*)act);
         KCK();
       }
     }
