@@ -272,7 +272,7 @@ __global__ void __launch_bounds__(256) kb_finish_max(const ACfl<T>* __restrict__
   if (threadIdx.x == 0) out[blockIdx.x] = m;
 }
 
-// solver! control per simulation (src/MultiLevelPoisson.jl:110-125): k_mg_init / k_mg_control on
+// solver! control per simulation (src/MultiLevelPoisson.jl:110-125): the start and control on
 // each simulation's scalars, plus the iteration count and the "still iterating" flag.
 struct ACtl {
   double* dsc;

@@ -2976,15 +2976,15 @@ __global__ void __launch_bounds__(256) k_body_metrics(Geo g, Box b, DBodies bs, 
   if (threadIdx.x == 0 && threadIdx.y == 0)
     for (int q = 0; q < 12; ++q) partial[block_linear_id() + q * pstride] = acc[q];
 }
-// one workgroup per row q of partial: out[q] = Σ partial[q·pstride .. q·pstride + np)
+// one workgroup per row q of partial: Σ partial[q·pstride .. q·pstride + np), posted to the host
 __global__ void __launch_bounds__(256) k_finish_rows(const double* __restrict__ partial, int64_t np, int64_t pstride,
-                                                     double* __restrict__ out) {
+                                                     double* __restrict__ host) {
   double acc = 0;
   const double* r = partial + blockIdx.x * pstride;
 #pragma unroll 16
   for (int64_t q = threadIdx.x; q < np; q += blockDim.x) acc += r[q];
   const double s = block_sum(acc);
-  if (threadIdx.x == 0) out[blockIdx.x] = s;
+  if (threadIdx.x == 0) host_post(host, HOST_ROW0 + (int)blockIdx.x, s);
 }
 
 // MeanFlow update! blend (src/Metrics.jl:234-240) with weight e: P = e·p + (1−e)·P, U likewise,
@@ -3026,11 +3026,6 @@ template <class T>
 __global__ void k_mg_init(const double* __restrict__ dsc, T* __restrict__ st) {
   if (threadIdx.x == 0) mg_init_state<T>(dsc[1], st);
 }
-template <class T>
-__global__ void k_mg_control(double* __restrict__ dsc, T* __restrict__ st) {
-  if (threadIdx.x == 0) mg_control_state<T>(dsc[1], dsc, st);
-}
-
 // ---- mixed precision: FP32 V-cycles inside an FP64 defect-correction loop ----
 // The outer residual r = z − A·x is evaluated in double from the FP32 coefficients and an FP64
 // solution x64, then rounded to T for the V-cycle, which solves A·c = r for the correction c
@@ -3129,10 +3124,12 @@ __global__ void __launch_bounds__(256) k_residual64(Geo g, ZT t, LRows<T> LR, co
   if (threadIdx.x == 0 && threadIdx.y == 0) { partial[blockIdx.x] = s1; partial[nb + blockIdx.x] = s2; }
 }
 // Σr, the mean s = Σr/N and Σ(r − s)² = Σr² − N·s² (the mean is removed when |s| > 2eps(T),
-// src/Poisson.jl:95-97): dsc[0] = Σr, dsc[1] = the residual norm; st[0] = (T)s, st[1] = flag.
+// src/Poisson.jl:95-97): dsc[0] = Σr, dsc[1] = the residual norm; st[0] = (T)s, st[1] = flag; then the
+// solver's start or its control (FinMode).
 template <class T>
 __global__ void __launch_bounds__(1024) k_finish_sum2(const double* __restrict__ partial, int64_t nb,
-                                                      double* __restrict__ dsc, T* __restrict__ st, double ninside) {
+                                                      double* __restrict__ dsc, T* __restrict__ st, double ninside,
+                                                      int mode, double* __restrict__ host) {
   double a = 0, b = 0;
 #pragma unroll 4
   for (int64_t q = threadIdx.x; q < nb; q += blockDim.x) { a += partial[q]; b += partial[nb + q]; }
@@ -3142,9 +3139,9 @@ __global__ void __launch_bounds__(1024) k_finish_sum2(const double* __restrict__
     const double s = a / ninside;
     const bool sub = fabs(s) > 2.0 * (double)eps_t<T>();
     dsc[0] = a;
-    dsc[1] = sub ? b - ninside * s * s : b;
     st[0] = (T)s;
     st[1] = sub ? T(1) : T(0);
+    fin_apply<T>(mode, sub ? b - ninside * s * s : b, dsc + 1, st, ninside, dsc, host);
   }
 }
 // r −= s (when flagged), ϵ = r·iD, correction c = 0: the V-cycle's start on the defect

@@ -738,7 +738,7 @@ struct MG {
   static constexpr int64_t chain_cells = 4096;
 
   // mode 0: Σ into dsc[slot]; 1: also the mean and its flag (tsc[0..1]); 2 and 3 (slot 1): then the
-  // solver's init or ω control on the device state, as k_mg_init / k_mg_control would
+  // solver's init or ω control on the device state, as k_mg_init would, or its control
   // the partials start at B->partial + poff
   double finish_sum(int64_t np, int slot, int mode = 0, double ninside = 1, int64_t poff = 0) {
     hipLaunchKernelGGL(k_finish_sum<T>, dim3(1), dim3(1024), 0, st, (const double*)B->partial + poff, np, B->dsc + slot,
@@ -1488,7 +1488,8 @@ struct MG {
   // Mixed precision (WL_SOLVER_MIXED): each iteration runs the FP32 V-cycle and finest smooth! on
   // the defect r (level-0 x is the correction c, from 0), then x64 += c and r = z − A·x64 in FP64
   // (k_residual64); ω adapts on, and the loop stops on, that FP64 Σr² (src/MultiLevelPoisson.jl:
-  // 108-127 otherwise).  Expects x64[x64cur] and dsc[1] from the projection's first pass.
+  // 108-127 otherwise).  Expects x64[x64cur], dsc[1] and the solver's start from the projection's
+  // first pass.
   void ensure_x64() {
     for (auto& b : x64)
       if (!b) b = dalloc<double>(lv[0].g.n);
@@ -1501,9 +1502,9 @@ struct MG {
   T* c_alt = nullptr;
   bool mixed_prepped = false;  // the last FP64 residual pass formed ϵ and c
   bool mixed_fused() const { return perdir == 0 && lv[0].ej != nullptr; }
-  void finish_sum2(int64_t nb) {
+  void finish_sum2(int64_t nb, int mode = FIN_INIT) {
     hipLaunchKernelGGL(k_finish_sum2<T>, dim3(1), dim3(1024), 0, st, (const double*)B->partial, nb, B->dsc, (T*)B->tsc,
-                       (double)ninside(lv[0].g));
+                       (double)ninside(lv[0].g), mode, B->host);
     KCK();
   }
   int mixed_loop(double tol, int itmx, std::vector<double>* hist) {
@@ -1511,9 +1512,7 @@ struct MG {
     ZT bi = zt_inside(p.g);
     const int64_t nb = zt_blocks(bi);
     const T* w = (const T*)B->tsc + 3;
-    hipLaunchKernelGGL(k_mg_init<T>, dim3(1), dim3(64), 0, st, (const double*)B->dsc, (T*)B->tsc);
-    KCK();
-    if (hist) hist->push_back((double)(T)read_dsc(1));
+    if (itmx <= 0 && hist) hist->push_back((double)(T)read_dsc(1));
     T* const x0 = p.x;  // the level-0 x the loop ends on (c may sit in c_alt meanwhile)
     int n = 0;
     while (n < itmx) {
@@ -1577,13 +1576,13 @@ struct MG {
       }
       x64cur = 1 - x64cur;
       perbc(p.g, x64[x64cur]);
-      finish_sum2(nb);
-      hipLaunchKernelGGL(k_mg_control<T>, dim3(1), dim3(64), 0, st, B->dsc, (T*)B->tsc);
-      KCK();
-      HIPCK(hipMemcpyAsync(B->hsc, B->dsc, 8 * sizeof(double), hipMemcpyDeviceToHost, st));
-      HIPCK(hipStreamSynchronize(st));
-      const T rnew = (T)B->hsc[1];
-      if (hist) hist->push_back((double)rnew);
+      host_unset(*B, HOST_R2);
+      finish_sum2(nb, FIN_CONTROL);
+      const T rnew = (T)host_wait(*B, HOST_R2, st);
+      if (hist) {
+        if (n == 0) hist->push_back(B->host[HOST_R2_OLD]);
+        hist->push_back((double)rnew);
+      }
       n++;
       if ((double)rnew < tol) break;
       if (!std::isfinite(rnew)) {
@@ -2362,8 +2361,8 @@ struct FlowT : FlowBase {
     DBodies bs = to_dbodies(b, nb);
     metrics_run(bs, x0, out, part);
   }
-  // k_body_metrics writes 12 rows of np block partials into part, k_finish_rows sums each row
-  // into part[12·np ..]; allocates nothing
+  // k_body_metrics writes 12 rows of np block partials into part, k_finish_rows sums each row and posts
+  // it to the host; allocates nothing
   void metrics_run(const DBodies& bs, const double* x0, double* out, double* part) {
     Box bi = box_inside(g);
     const int64_t np = nblocks(bi);
@@ -2372,10 +2371,10 @@ struct FlowT : FlowBase {
     hipLaunchKernelGGL(k_body_metrics<T>, grid_of(bi), kBlock, 0, st, g, bi, bs, (const T*)p, (const T*)u,
                        (T)desc.nu, x, part, np);
     KCK();
-    hipLaunchKernelGGL(k_finish_rows, dim3(12), dim3(256), 0, st, (const double*)part, np, np, part + 12 * np);
+    for (int q = 0; q < 12; ++q) host_unset(B, HOST_ROW0 + q);
+    hipLaunchKernelGGL(k_finish_rows, dim3(12), dim3(256), 0, st, (const double*)part, np, np, B.host);
     KCK();
-    HIPCK(hipMemcpyAsync(out, part + 12 * np, 12 * sizeof(double), hipMemcpyDeviceToHost, st));
-    HIPCK(hipStreamSynchronize(st));
+    for (int q = 0; q < 12; ++q) out[q] = host_wait(B, HOST_ROW0 + q, st);
   }
   hipStream_t stream() const override { return st; }
 };
