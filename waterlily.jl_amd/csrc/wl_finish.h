@@ -36,13 +36,14 @@ __device__ __forceinline__ void mg_control_state(double r2sum, double* __restric
 // blocks' partials take what the launch takes, 139 -> 143 us at 64x64; with thousands of blocks the
 // fences' cache write-backs cost more than the pass, 870 -> 1610 us at 256x128x128.)
 constexpr unsigned long long HOST_UNSET = 0xfff8a5a5a5a5a5a5ull;
-enum HostSlot { HOST_R2 = 0, HOST_R2_OLD = 1, HOST_MAX = 2, HOST_ROWS = 3, HOST_ROW0 = 8, HOST_SLOTS = 20 };
+enum HostSlot { HOST_R2 = 0, HOST_R2_OLD = 1, HOST_MAX = 2, HOST_ROWS = 3, HOST_DONE = 4, HOST_ROW0 = 8, HOST_SLOTS = 20 };
 __device__ __forceinline__ void host_post(double* __restrict__ host, int slot, double v) {
   unsigned long long b = (unsigned long long)__double_as_longlong(v);
   if (b == HOST_UNSET) b = 0x7ff8000000000000ull;
   __hip_atomic_store((unsigned long long*)host + slot, b, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+__global__ void k_post_done(double* __restrict__ host) { host_post(host, HOST_DONE, 1.0); }
 // What a control decides besides ω: whether another iteration follows (the host's own tests, with its
 // tolerance; last: the iteration limit is reached).  A launch that is issued before the host has read
 // Σr² carries a Gate and ends at once where the decision was the other one.

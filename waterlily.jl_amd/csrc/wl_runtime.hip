@@ -1832,7 +1832,14 @@ struct FlowT : FlowBase {
     mu1_dirty = false;
     crows_ok = false;
     mg.lv[0].lrow_ok = false;
-    sync();
+    wait_done();
+  }
+  // the stream's end, as the solver's results are waited for
+  void wait_done() {
+    host_unset(B, HOST_DONE);
+    hipLaunchKernelGGL(k_post_done, dim3(1), dim3(1), 0, st, B.host);
+    KCK();
+    (void)host_wait(B, HOST_DONE, st);
   }
   uint8_t* vrows() const { return rows + (int64_t)g.N[1] * g.N[2]; }
   uint8_t* crows() const { return rows + 2 * (int64_t)g.N[1] * g.N[2]; }
@@ -1870,7 +1877,7 @@ struct FlowT : FlowBase {
   }
   void pois_update() override {
     mg.update();
-    sync();
+    wait_done();
   }
 
   // convection tiles: 63 output columns and CBY-1 output rows per block (overlapping)
