@@ -222,13 +222,16 @@ def copy_calibration(nbytes=1 << 30, reps=5):
 
 # rocprofv3 kernel names -> the library's profiler keys (level 0 = the largest dispatch of a name)
 PROF_KEYS = {"k_inc_restrict_full": "inc_restrict", "k_mg_tail": "mg_tail", "k_mg_tail_lds": "mg_tail", "k_bdim2": "bdim2", "k_residual": "residual", "k_submean_l2": "submean_l2",
-             "k_submean_l2_cond": "submean_l2",
              "k_inc_restrict": "inc_restrict", "k_gs_half": "gs_half", "k_increment": "increment",
              "k_prolong_inc": "prolong_inc", "k_eps_init": "eps_init", "k_correct": "correct", "k_cfl": "cfl",
              # the x-pair multigrid kernels (two cells per lane)
              "k_gs_half2": "gs_half", "k_increment2": "increment", "k_inc_restrict2": "inc_restrict",
              "k_prolong_inc2": "prolong_inc", "k_gs_half_s": "gs_half", "k_gs_dbl": "gs_dbl", "k_smooth4": "smooth4",
              "k_residual64": "residual64",
+             # large 3D levels; a level's up-leg; the coarse tail of few pairs; the residual's second stage
+             "k_lean_gs": "gs_half", "k_lean_gs_first": "gs_first", "k_lean_restrict": "inc_restrict",
+             "k_lean_prolong": "prolong_inc", "k_lean_increment": "increment", "k_up": "up",
+             "k_mg_tail_fast": "mg_tail", "k_mean_l2": "submean_l2",
              # BDIM!'s rows the convection kernel leaves (a list of rows), and their flags
              "k_bdim2_rows": "bdim2", "k_conv_rows": "conv_rows", "k_copy_exit_plane": "exit_plane"}
 
