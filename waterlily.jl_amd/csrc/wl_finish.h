@@ -108,13 +108,16 @@ __device__ __forceinline__ void fin_total(const double* partial, int64_t np, int
   for (int k = 0; k < N; ++k)
 #pragma unroll
     for (int j = 0; j < 4; ++j) a[k][j] = 0;
-#pragma unroll 2
+#pragma unroll 4
   for (int64_t q = t; q < np; q += 1024)
 #pragma unroll
     for (int k = 0; k < N; ++k)
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (q + 256 * j < np) a[k][j] += partial[k * stride + q + 256 * j];
+      for (int j = 0; j < 4; ++j) {  // no branch between the loads: one beyond np reads slot 0 and adds 0
+        const bool in = q + 256 * j < np;
+        const double v = partial[k * stride + (in ? q + 256 * j : 0)];
+        a[k][j] += in ? v : 0.0;
+      }
 #pragma unroll
   for (int k = 0; k < N; ++k)
 #pragma unroll

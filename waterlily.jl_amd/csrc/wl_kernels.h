@@ -1224,7 +1224,7 @@ __global__ void __launch_bounds__(256) k_submean_l2(Geo g, ZT t, LRows<T> LR, T*
 // launch goes on with it: each block walks the blocks b = blockIdx.x + k·gridDim.x of the nb-block
 // launch above (same tiles, same partial slots), and the one that ends last adds up the new Σr².
 // One launch for the three that add, subtract where flagged, and add again: 8 -> 3.6 us at 192x128,
-// 14 -> 10 us at 256x128x128.
+// 14 -> 5 us at 256x128x128.
 template <class T>
 __global__ void __launch_bounds__(256) k_mean_l2(Geo g, ZT t, LRows<T> LR, T* __restrict__ r, T* __restrict__ e,
                                                  double* partial, int nb, int mode, double ninside, double* dsc, T* st,
