@@ -2263,9 +2263,11 @@ struct FlowT : FlowBase {
     if (use_net) warm_guess();
     const ZT ba = make_zt_short(box_all(g), 8);
     auto correct = [&](Gate gate) {
-      ProfScope ps(&prof, st, "correct", 0, (double)sizeof(T) * (2 * g.n + 2 * D * ncells_inside(g)));
-      hipLaunchKernelGGL(k_correct<T>, zt_grid(ba), kBlock, 0, st, g, ba, u, mg.lr(0), (const T*)xw, p, dt, gate);
-      KCK();
+      {
+        ProfScope ps(&prof, st, "correct", 0, (double)sizeof(T) * (2 * g.n + 2 * D * ncells_inside(g)));
+        hipLaunchKernelGGL(k_correct<T>, zt_grid(ba), kBlock, 0, st, g, ba, u, mg.lr(0), (const T*)xw, p, dt, gate);
+        KCK();
+      }
       apply_bc_u(t1, gate);
     };
     bool corrected = false;
