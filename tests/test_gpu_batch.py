@@ -91,3 +91,21 @@ def test_batch_large_3d_member(wl):
     for a, c in zip(batched, single):
         assert a.flow.Δt == c.flow.Δt and a.pois.n == c.pois.n
     say("  n =", [a.pois.n[-2:] for a in batched])
+
+
+@pytest.mark.parametrize("T", [np.float32, np.float64])
+def test_batch_of_odd_coarse_levels(wl, T):
+    """3D members whose coarse levels' cells sum to no multiple of 4 (the tail's image is rounded up to
+    whole vectors), beside one whose do, in either order of sizes: against stepping each alone."""
+    say("case: batch of 3D members with odd coarse levels,", T.__name__)
+    shapes = [(48, 48, 48), (8, 9, 9), (32, 16, 17), (64, 32, 32)]
+    sims = [[wl.Simulation(n, (1, 0, 0), min(n) / 3, ν=0.02, body=wl.Sphere(tuple(v / 2 for v in n), min(n) / 6), T=T)
+             for n in shapes] for _ in range(2)]
+    b = wl.Batch(sims[0])
+    for k in range(3):
+        b.step()
+        for s in sims[1]:
+            wl.sim_step(s, remeasure=False)
+        for a, c in zip(*sims):
+            for name in ("u", "p"):
+                assert np.array_equal(a.flow.get(name), c.flow.get(name)), (k, name, a.flow.N)

@@ -3,6 +3,7 @@
 //
 // Included by wl_kernels.h after the per-cell pieces it uses (LRows, lcell, pro_map, TailDesc).
 #pragma once
+#include "wl_tail.h"
 
 namespace wl {
 
@@ -421,14 +422,6 @@ __global__ void __launch_bounds__(1024) k_mg_tail_lds(TailDesc<T> d, const T* __
 // other threads read (ϵ, the residuals a restriction sums, the coarse x); the L, D and 1/D of all
 // levels lie in one image in memory, formed when L changes (k_level_tables), so one round of loads
 // brings them in.
-struct TailLv {           // one level; built on the host, read with scalar loads
-  int N0, N1, N2;
-  int s1, s2, n, cm;
-  int lx, ly;             // log2 of the threads along x (pairs) and y
-  int oL, oD, oI;         // LDS element offsets: L (D arrays of n), D, 1/D ...
-  int oR, oX, oE;         // ... r, x, ϵ
-  int small;              // run by the first wave alone
-};
 template <class T>
 struct TailFast {
   int n, perdir, exact, nimg;  // levels; image elements

@@ -944,11 +944,11 @@ struct MG {
     if (l2) finish_sum(zt_blocks(b), 1, fmode);
   }
 
-  // LDS bytes the levels l..end need in the coarse tail (L, x, r, ϵ of each)
-  int64_t tail_bytes(int l) const {
-    int64_t b = 0;
-    for (size_t k = l; k < lv.size(); ++k) b += (int64_t)(lv[k].g.D + 5) * lv[k].g.n * (int64_t)sizeof(T);
-    return b;
+  // LDS bytes of a coarse tail over the levels l..end: the general one, or k_mg_tail_fast
+  int64_t tail_bytes(int l, bool fast) const {
+    int64_t n = 0;
+    for (size_t k = l; k < lv.size(); ++k) n += lv[k].g.n;
+    return (int64_t)tail_lds_bytes(lv[l].g.D, n, fast, sizeof(T));
   }
   // First level run by the single-workgroup coarse tail: the first level (>= 1) from which every
   // coarser level fits the tail's LDS image; WL_TAIL_CELLS (cells of the first tail level) makes
@@ -967,7 +967,7 @@ struct MG {
     return (int)std::min<int64_t>(t, 1 << 20);
   }
   bool tail_fast(int l) const {
-    return fold_coarse_inc && tail_threads(lv[l].g) <= TAIL_FAST_PAIRS && tail_bytes(l) <= TAIL_LDS_BYTES;
+    return fold_coarse_inc && tail_threads(lv[l].g) <= TAIL_FAST_PAIRS && tail_bytes(l, true) <= TAIL_LDS_BYTES;
   }
   int tail_start(bool* in_lds) const {
     const int64_t cells = tail_cells;
@@ -982,7 +982,7 @@ struct MG {
       return -1;
     }
     for (size_t l = 1; l < lv.size(); ++l)
-      if (tail_bytes((int)l) <= TAIL_LDS_BYTES) { *in_lds = true; return (int)l; }
+      if (tail_bytes((int)l, false) <= TAIL_LDS_BYTES) { *in_lds = true; return (int)l; }
     return -1;
   }
   // the fast tail's image of L, D and 1/D (k_level_tables), formed with L in update()
@@ -992,7 +992,6 @@ struct MG {
     std::memset(&d, 0, sizeof(d));
     d.n = (int)lv.size() - Lt;
     d.perdir = perdir;
-    int o = 0;
     for (int k = 0; k < d.n; ++k) {
       const Geo& g = lv[Lt + k].g;
       TailLv& q = d.lv[k];
@@ -1000,28 +999,12 @@ struct MG {
       q.s1 = (int)g.s[1]; q.s2 = (int)g.s[2]; q.n = (int)g.n; q.cm = lv[Lt + k].cmask;
       q.lx = log2_up_h((g.N[0] - 1) / 2); q.ly = log2_up_h(g.N[1] - 2);
       q.small = tail_threads(g) <= TAIL_WAVE_PAIRS;
-      q.oL = o;
-      q.oD = o + g.D * q.n;
-      q.oI = q.oD + q.n;
-      o = q.oI + q.n;
     }
-    o = (o + 3) & ~3;
-    d.nimg = o;
-    for (int k = 0; k < d.n; ++k) {
-      TailLv& q = d.lv[k];
-      q.oR = o;
-      q.oX = o + q.n;
-      q.oE = q.oX + q.n;
-      o = q.oE + q.n;
-    }
+    tail_fast_layout(lv[Lt].g.D, d.lv, d.n, &d.nimg);
     d.img = tail_img;
     d.r = lv[Lt].r;
     d.x = lv[Lt].x;
     return d;
-  }
-  static size_t tail_desc_lds(const TailFast<T>& d) {
-    const TailLv& q = d.lv[d.n - 1];
-    return (size_t)(q.oE + q.n) * sizeof(T);
   }
   bool exact_coarsest = false;  // set by the mixed-precision loop around its V-cycles
   bool coarse_pcg = false;      // WL_COARSE_PCG=1: that coarsest level by FP64 pcg! instead of GS-RB
@@ -1029,11 +1012,12 @@ struct MG {
     if (in_lds && tail_fast(Lt)) {
       TailFast<T> f = tail_desc(Lt);
       f.exact = exact_coarsest ? (coarse_pcg ? 2 : 1) : 0;
+      const size_t lds = (size_t)tail_bytes(Lt, true);
       ProfScope ps(P, st, "mg_tail", Lt, 0.0);
       if (lv[Lt].g.D == 3)
-        hipLaunchKernelGGL((k_mg_tail_fast<T, 3>), dim3(1), dim3(TAIL_FAST_PAIRS), tail_desc_lds(f), st, f, w);
+        hipLaunchKernelGGL((k_mg_tail_fast<T, 3>), dim3(1), dim3(TAIL_FAST_PAIRS), lds, st, f, w);
       else
-        hipLaunchKernelGGL((k_mg_tail_fast<T, 2>), dim3(1), dim3(TAIL_FAST_PAIRS), tail_desc_lds(f), st, f, w);
+        hipLaunchKernelGGL((k_mg_tail_fast<T, 2>), dim3(1), dim3(TAIL_FAST_PAIRS), lds, st, f, w);
       KCK();
       return;
     }
@@ -1056,7 +1040,7 @@ struct MG {
     ProfScope ps(P, st, "mg_tail", Lt, 0.0);
     if (in_lds) {
       // a standalone MultiLevelPoisson keeps its coarse levels' whole state
-      const size_t lds = (size_t)(off * sizeof(T));
+      const size_t lds = (size_t)tail_bytes(Lt, false);
       if (lv[Lt].g.D == 3) {
         if (fold_coarse_inc) hipLaunchKernelGGL((k_mg_tail_lds<T, 3, false>), dim3(1), dim3(1024), lds, st, d, w);
         else hipLaunchKernelGGL((k_mg_tail_lds<T, 3, true>), dim3(1), dim3(1024), lds, st, d, w);
@@ -2647,9 +2631,9 @@ struct BatchT : BatchBase {
           t.d.lv[k].off = off;
           off += (int64_t)(q.g.D + 5) * q.g.n;
         }
-        tail_lds = std::max(tail_lds, (size_t)(off * sizeof(T)));
         t.wp = (const T*)F[s]->B.tsc + 3;
         t.fast = mg.tail_fast(Lt[s]) ? 1 : 0;
+        tail_lds = std::max(tail_lds, (size_t)mg.tail_bytes(Lt[s], t.fast != 0));
         if (t.fast) t.f = mg.tail_desc(Lt[s]);
         a.push_back(t);
         sims.push_back(s);
