@@ -183,3 +183,29 @@ def test_measured_fields_and_levels(wl, n, perdir, T):
     while l + 1 < len(ml.levels):
         L, l = restrict_l(L, perdir), l + 1
         assert np.array_equal(ml.get("L", l), L), l
+
+
+@pytest.mark.parametrize("T", [np.float32, np.float64])
+@pytest.mark.parametrize("how", ["upload", "measure"])
+def test_lean_follows_mu0_without_update(wl, how, T, monkeypatch):
+    """μ₀ changed without update!: the lean passes' 1/D is that of the L they read, as in the passes
+    that form it, with the row flags and without (WL_LROWS=0)."""
+    print("case: lean after a change of mu0 alone", how, T.__name__, flush=True)
+    n, got = (144, 56, 48), []
+    moved = wl.Sphere((60.5, 26.1, 23.9), 9.1)  # (the coarse levels keep the other body's)
+    mu0 = wl.Simulation(n, (1, 0, 0), 18, ν=0.02, body=moved, T=T).flow.get("mu0")
+    for lean, rows in (("0", "1"), ("0", "0"), ("2", "1"), ("2", "0")):
+        monkeypatch.setenv("WL_LEAN", lean)
+        monkeypatch.setenv("WL_LROWS", rows)
+        sim = wl.Simulation(n, (1, 0, 0), 18, ν=0.02, body=wl.Sphere((60.3, 26.0, 24.0), 9), T=T)
+        wl.sim_step(sim, remeasure=False)
+        if how == "upload":
+            sim.flow.set("mu0", mu0)
+        else:
+            wl.measure_flow(sim.flow, moved)
+        for _ in range(2):
+            wl.sim_step(sim, remeasure=False)
+        got.append([sim.flow.get("u"), sim.flow.get("p"), list(sim.pois.n)])
+    for g in got[1:]:
+        for a, b in zip(got[0], g):
+            assert np.array_equal(a, b)

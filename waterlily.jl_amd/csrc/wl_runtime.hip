@@ -234,6 +234,7 @@ struct Level {
   // coarse level the colour-split ϵ (the finest level's is MG::se)
   T *r2 = nullptr, *iD = nullptr, *se = nullptr;
   uint8_t* lseg = nullptr;  // per row and 128 cells: bits, uniform, fast (k_seg_*)
+  bool lean_ok = false;     // iD (and lseg, with lrow_ok) matches the current L
   SplitG sg{0, 0};
 };
 
@@ -506,7 +507,7 @@ struct MG {
     };
     for (int l = 0; l < (int)lv.size(); ++l) {
       Level<T>& p = lv[l];
-      if (!all && p.lrow_ok) continue;
+      if (!all && tables_ok(p)) continue;
       if (l == 0) ++lrow_epoch0;
       const bool img = image && l >= Lt;
       p.lrow_ok = false;
@@ -531,6 +532,7 @@ struct MG {
     Box b = box_inside(p.g);
     hipLaunchKernelGGL(k_diag<T>, grid_of(b), kBlock, 0, st, p.g, b, (const T*)p.L, p.iD, 1);
     KCK();
+    p.lean_ok = true;
     if (!use_lrows) return;
     const int ns = lean_nseg(p.g);
     const int64_t nk = (int64_t)p.g.N[1] * p.g.N[2] * ns;
@@ -544,10 +546,11 @@ struct MG {
                        (const uint8_t*)p.lseg + nk, p.lseg + 2 * nk);
     KCK();
   }
+  bool tables_ok(const Level<T>& p) const { return (p.lrow_ok || !use_lrows) && (p.lean_ok || !p.iD); }
+  void l_changed(int l) { lv[l].lrow_ok = lv[l].lean_ok = false; }  // by anything but update()
   void ensure_lrows() {
-    if (!use_lrows) return;
     for (auto& p : lv)
-      if (!p.lrow_ok) {
+      if (!tables_ok(p)) {
         build_tables(false);
         return;
       }
@@ -1815,7 +1818,7 @@ struct FlowT : FlowBase {
     KCK();
     mu1_dirty = false;
     crows_ok = false;
-    mg.lv[0].lrow_ok = false;
+    mg.l_changed(0);
     wait_done();
   }
   // the stream's end, as the solver's results are waited for
@@ -1846,7 +1849,7 @@ struct FlowT : FlowBase {
   }
   void field_uploaded(int field) override {
     if (field == WL_MU1 || field == WL_V) mu1_dirty = true;
-    if (field == WL_MU0) mg.lv[0].lrow_ok = false;  // L of the finest level is μ₀
+    if (field == WL_MU0) mg.l_changed(0);  // L of the finest level is μ₀
   }
   void mu1_rows() {
     const int64_t nr = (int64_t)g.N[1] * g.N[2];
