@@ -209,3 +209,31 @@ def test_lean_follows_mu0_without_update(wl, how, T, monkeypatch):
     for g in got[1:]:
         for a, b in zip(got[0], g):
             assert np.array_equal(a, b)
+
+
+def launches(flow, run):
+    """The profiled (name, level, bytes) of what `run` launches."""
+    flow.profile(True)
+    run()
+    got = {(k["name"], k["level"], k["bytes_per_launch"]) for k in flow.profile_read()}
+    flow.profile(False)
+    return got
+
+
+@pytest.mark.parametrize("mode", ["plain", "mixed"])
+@pytest.mark.parametrize("lean", ["0", "2"])
+def test_autotune_times_the_flows_own_launches(wl, lean, mode, monkeypatch):
+    """The tile autotuner of a 3D flow times launches that its steps make, and with the lean passes on
+    the finest level none of that level, which take no target."""
+    print("case: autotune", lean, mode, flush=True)
+    monkeypatch.setenv("WL_LEAN", lean)
+    sim = wl.Simulation((272, 56, 48), (1, 0, 0), 18, ν=0.02, body=wl.Sphere((60.3, 26.0, 24.0), 9))
+    sim.pois.set_solver(mode=wl.WL_SOLVER_MIXED if mode == "mixed" else wl.WL_SOLVER_PLAIN)
+    for _ in range(2):
+        wl.sim_step(sim, remeasure=False)
+    u, p = sim.flow.u, sim.flow.p
+    timed = launches(sim.flow, lambda: sim.flow.autotune(1))
+    assert np.array_equal(sim.flow.u, u) and np.array_equal(sim.flow.p, p)
+    stepped = launches(sim.flow, lambda: wl.sim_step(sim, remeasure=False))
+    assert timed and timed <= stepped, timed - stepped
+    assert (min(k[1] for k in timed) == 0) == (lean == "0" or mode == "mixed")

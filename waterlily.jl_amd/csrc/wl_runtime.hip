@@ -1134,6 +1134,9 @@ struct MG {
     }
     return done;
   }
+  // whether the up-leg leaves coarse level c with its smooth! and increment! done, by the tail (from Lt)
+  // or by k_up on top of such a level; elsewhere its increment! is folded into the prolongation
+  bool smoothed(int c, int Lt) const { return Lt > 0 && (c >= Lt || (up_ok(c) && smoothed(c + 1, Lt))); }
   // k_up in place of the separate launches of a level: a flow's own solver (nobody reads the level's
   // r and ϵ afterwards), levels below up_cells cells.
   bool up_ok(int l) const {
@@ -1276,15 +1279,19 @@ struct MG {
 
   // Tile autotuner: the blocks-in-flight targets of the GS half sweeps and of the restriction /
   // prolongation kernels (kernels without reductions, whose results do not depend on the tiling),
-  // chosen by timing `reps` level-0 launches of each candidate with HIP events.  The buffers the
-  // timed launches write are saved first and restored after, so the solver state is unchanged.
+  // chosen by timing `reps` launches of each candidate with HIP events, on the finest level that takes
+  // the target: level 0, or under lean passes, which take none, the first other level (the half
+  // sweeps' target is level 0's alone and stays as it is).  lean_run: the flow's projections run the
+  // lean passes where the solver has them.  (A 2D flow's own steps take k_up on level 0; its separate
+  // passes are timed for the batches it may join.)  The buffers the timed launches write are saved
+  // first and restored after, so the solver state is unchanged.
   int zt_gs = 0, zt_rp = 0;  // 0: the defaults
   int tgt_gs() const { return zt_gs ? zt_gs : zt_target_default(); }
   // the half sweeps' target on level l: the autotuner times level 0 only; the coarser levels take
   // 2048 (level 1 of 512x256x256: 14.7 us per half sweep, against 17.3 at 1024 and 15.9 at 8192)
   int tgt_gs_at(int l) const { return l == 0 ? tgt_gs() : 2048; }
   int tgt_rp() const { return zt_rp ? zt_rp : 2 * zt_target_default(); }
-  void autotune(int reps, const T* w) {
+  void autotune(int reps, const T* w, bool lean_run) {
     if (lv.size() < 2 || reps < 1) return;
     free_graphs();  // captured iterations hold the old tile shapes
     // the kernels a projection runs: with the colour-split ϵ when the flow's projections use it
@@ -1293,11 +1300,16 @@ struct MG {
       MG* m;
       ~SplitScope() { if (m) m->split_end(); }
     } split_scope{sp ? this : nullptr};
-    if (sp) split_begin(true);
-    Level<T>& f = lv[0];
-    Level<T>& c = lv[1];
+    if (sp) split_begin(lean_run);
+    bool in_lds = false;
+    const int Lt = tail_start(&in_lds), down_end = Lt > 0 ? Lt : (int)lv.size() - 1;
+    int l = 0;
+    while (l < down_end && lean(l)) ++l;
+    if (l == down_end) return;
+    Level<T>& f = lv[l];
+    Level<T>& c = lv[l + 1];
     T* bufs[6] = {f.e, f.r, f.x, c.e, c.r, c.x};
-    const int64_t ns[6] = {sp ? 2 * sg.H : f.g.n, f.g.n, f.g.n, c.g.n, c.g.n, c.g.n};
+    const int64_t ns[6] = {sp && l == 0 ? 2 * sg.H : f.g.n, f.g.n, f.g.n, c.g.n, c.g.n, c.g.n};
     int64_t tot = 0;
     for (int64_t v : ns) tot += v;
     T* save = dalloc<T>(tot);
@@ -1328,19 +1340,21 @@ struct MG {
       static const int cands[] = {1024, 2048, 4096, 8192, 16384};
       float best = 1e30f;
       int pick = 0;
-      for (int cnd : cands) {
-        zt_gs = cnd;
-        const float ms = timed([&] { if (lean(0)) gs_lean(0); else gs_sweeps(0); });
-        if (ms < best) { best = ms; pick = cnd; }
+      if (l == 0) {
+        for (int cnd : cands) {
+          zt_gs = cnd;
+          const float ms = timed([&] { gs_sweeps(0); });
+          if (ms < best) { best = ms; pick = cnd; }
+        }
+        zt_gs = pick;
       }
-      zt_gs = pick;
       best = 1e30f;
       pick = 0;
       for (int cnd : cands) {
         zt_rp = cnd;
         const float ms = timed([&] {
-          restrict_level(0);
-          if (lean(0)) prolong_lean(1, w, lean(1)); else prolong_level(1, w);
+          restrict_level(l);
+          if (l == 0 || !up_ok(l)) prolong_level(l + 1, w, fold_coarse_inc && !smoothed(l + 1, Lt));
         });
         if (ms < best) { best = ms; pick = cnd; }
       }
@@ -2280,7 +2294,7 @@ struct FlowT : FlowBase {
     sync();
     if (mu1_dirty) mu1_rows();
     mg.ensure_lrows();
-    mg.autotune(reps, (const T*)B.tsc + 3);
+    mg.autotune(reps, (const T*)B.tsc + 3, mode == WL_SOLVER_PLAIN && !net);
     if (targets) { targets[0] = mg.tgt_gs(); targets[1] = mg.tgt_rp(); }
   }
   // CFL(a) (src/Flow.jl:234-237) of the current u: min(10, 1/(max flux out of a cell + 5ν)),
