@@ -237,3 +237,33 @@ def test_autotune_times_the_flows_own_launches(wl, lean, mode, monkeypatch):
     stepped = launches(sim.flow, lambda: wl.sim_step(sim, remeasure=False))
     assert timed and timed <= stepped, timed - stepped
     assert (min(k[1] for k in timed) == 0) == (lean == "0" or mode == "mixed")
+
+
+@pytest.mark.parametrize("n,perdir", [((72, 40), ()), ((64, 33), ()), ((40, 32, 24), ()), ((136, 72), (2,)),
+                                      ((48, 32, 24), (3,)), ("batch", ())],
+                         ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else v)
+def test_up_cells_is_read_per_handle(wl, n, perdir, monkeypatch):
+    """WL_UP_CELLS=0 (every level by its separate passes) beside the default, one process: the same
+    V-cycles, u and p; k_up runs in the second alone."""
+    print("case: WL_UP_CELLS", n, perdir, flush=True)
+    shapes = [(72, 40), (128, 64)] if n == "batch" else [n]
+    got = []
+    for cells in ("0", None, "0"):
+        if cells is None:
+            monkeypatch.delenv("WL_UP_CELLS", raising=False)
+        else:
+            monkeypatch.setenv("WL_UP_CELLS", cells)
+        sims = [wl.Simulation(s, (1,) + (0,) * (len(s) - 1), min(s) / 3, ν=0.02, perdir=perdir,
+                              body=wl.Sphere(tuple(v / 2 - 0.3 for v in s), min(s) / 6)) for s in shapes]
+        keys = set()
+        if n == "batch":
+            b = wl.Batch(sims)
+            for _ in range(3):
+                b.step()
+        else:
+            for _ in range(3):
+                keys |= {k[0] for k in launches(sims[0].flow, lambda: wl.sim_step(sims[0], remeasure=False))}
+            assert bool(keys & {"up", "up_fin"}) == (cells is None), keys
+        got.append([v for s in sims for v in (s.flow.get("u"), s.flow.get("p"), list(s.pois.n))])
+    for a, b, c in zip(*got):
+        assert np.array_equal(a, b) and np.array_equal(a, c)

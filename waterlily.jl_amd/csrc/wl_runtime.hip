@@ -380,6 +380,8 @@ struct MG {
       use_split = !e8 || std::atoi(e8) != 0;
       const char* e9 = std::getenv("WL_LEAN");
       lean_sizes = e9 ? std::atoi(e9) : 1;
+      const char* e10 = std::getenv("WL_UP_CELLS");
+      up_cells = e10 ? (int64_t)std::atoll(e10) : (int64_t)-1;
     }
     lv.push_back(l0);
     if (!multilevel) return;
@@ -1142,16 +1144,9 @@ struct MG {
   bool up_ok(int l) const {
     const Geo& g = lv[l].g;
     for (int d = 0; d < g.D; ++d) if (g.N[d] < 4) return false;
-    return fold_coarse_inc && use_up && g.n <= up_cells(g.D);
+    return fold_coarse_inc && g.n <= (up_cells >= 0 ? up_cells : (g.D == 3 ? 100000 : (int64_t)1 << 40));
   }
-  bool use_up = true;
-  static int64_t up_cells(int D) {
-    static int64_t v = [] {
-      const char* e = std::getenv("WL_UP_CELLS");
-      return e ? (int64_t)std::atoll(e) : (int64_t)-1;
-    }();
-    return v >= 0 ? v : (D == 3 ? 100000 : (int64_t)1 << 40);
-  }
+  int64_t up_cells = -1;  // WL_UP_CELLS when the solver was built (-1: unset)
   bool fin_ok() const { return lv[0].g.D == 2 && up_ok(0) && fin_r != nullptr && perdir == 0; }
   T* fin_r = nullptr;  // the residual buffer k_up writes on the finest level; swapped with lv[0].r
   T* r_home = nullptr; // lv[0].r between solves
