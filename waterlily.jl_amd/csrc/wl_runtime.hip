@@ -1821,9 +1821,8 @@ struct FlowT : FlowBase {
     hipLaunchKernelGGL(k_fill<uint8_t>, dim3((unsigned)((2 * nr + 255) / 256)), dim3(256), 0, st, rows, 2 * nr,
                        (uint8_t)0);
     KCK();
-    Box ba = box_all(g);
-    hipLaunchKernelGGL(k_measure<T>, grid_of(ba), kBlock, 0, st, g, ba, bs, sigma, V, mu0, mu1, d2, (T)eps,
-                       desc.perdir_mask, rows);
+    hipLaunchKernelGGL(k_measure<T>, dim3((unsigned)((g.n + 255) / 256)), dim3(256), 0, st, g, bs, sigma, V, mu0, mu1,
+                       d2, (T)eps, desc.perdir_mask, rows);
     KCK();
     mu1_dirty = false;
     crows_ok = false;
