@@ -267,3 +267,32 @@ def test_up_cells_is_read_per_handle(wl, n, perdir, monkeypatch):
         got.append([v for s in sims for v in (s.flow.get("u"), s.flow.get("p"), list(s.pois.n))])
     for a, b, c in zip(*got):
         assert np.array_equal(a, b) and np.array_equal(a, c)
+
+
+@pytest.mark.parametrize("T", [np.float32, np.float64])
+@pytest.mark.parametrize("n,perdir", [((8, 8), ()), ((32, 32), ()), ((64, 64), ()), ((72, 56), ()), ((34, 68), ()),
+                                      ((64, 33), ()), ((64, 48), (1,)), ((8, 8, 8), ()), ((40, 24, 20), ()),
+                                      ((32, 16, 17), ()), ((32, 24, 40), (2, 3))],
+                         ids=lambda v: "x".join(map(str, v)) or "-")
+def test_standalone_multigrid_levels(wl, n, perdir, T):
+    """A MultiLevelPoisson of its own keeps every level's state (k_mg_tail_lds, whose passes take a cell
+    or a pair per thread): x and r of each level after two V-cycles, bit for bit.  The source is
+    antisymmetric, so no order of its sum removes a mean."""
+    print("case: standalone multigrid", n, perdir, T.__name__, flush=True)
+    rng, Ng, D = np.random.default_rng(11), tuple(v + 2 for v in n), len(n)
+    inner = (slice(1, -1),) * D
+    L = np.ones(Ng + (D,), T, order="F")
+    L[inner] = rng.uniform(0.1, 1.0, size=n + (D,))
+    bc_fill(L, perdir)
+    z = np.zeros(Ng, T, order="F")
+    v = rng.normal(size=n).astype(T)
+    z[inner] = v - np.flip(v)
+    x = np.zeros(Ng, T, order="F")
+    g, o = wl.MultiLevelPoisson(x, L, z, perdir=perdir), O.OPois(L, perdir=perdir, dtype=O.WL_F64 if T is np.float64 else O.WL_F32)
+    o.set("z", z)
+    wl.solver(g, tol=0, itmx=2)
+    o.solve(tol=0, itmx=2)
+    assert g.n == o.n and g.nlevels == o.nlevels
+    for l in range(g.nlevels):
+        for name in ("x", "r"):
+            assert np.array_equal(g.get(name, l), o.get(name, l)), (l, name)

@@ -83,10 +83,13 @@ __device__ __forceinline__ void tail_pcg(const SLev<T>& p, double (*cg)[TAIL_CG_
 //
 // What bounds it is latency: about 29 dependent passes of at most a few thousand cells, one
 // workgroup on an otherwise idle chip.  So
-//  - a thread owns x pairs: every half sweep updates one cell of each pair and no lane idles, and a
-//    level's pairs are dealt to the threads by shifts chosen from its own extents;
-//  - levels of at most 128 pairs run in the first wave alone, two pairs to a lane at most: the LDS
-//    serves a wave in order, so their passes need no barrier (the other waves wait at one);
+//  - in a half sweep a thread owns x pairs, one cell of which it updates, so no lane idles; in the other
+//    passes it owns one cell where the level has no more than threads (in pairs 35 us against 27.5 on
+//    32x32 and its three coarser levels), else pairs; both are dealt to the threads by shifts chosen
+//    from the level's own extents;
+//  - without KEEP, levels of at most 128 pairs run in the first wave alone, two pairs to a lane at most:
+//    the LDS serves a wave in order, so their passes need no barrier (the other waves wait at one);
+//    KEEP's passes over all cells take longer in one wave than the barriers cost (29 against 27.5 us);
 //  - without KEEP (a flow's own solver, whose coarse levels nobody reads) the last increment! of a
 //    level is x += ω·ϵ inside the fourth half sweep (its r is dead: the next V-cycle's restrict!
 //    overwrites it), nothing but the first level's x is stored, and only r and L are loaded.
@@ -122,6 +125,21 @@ __device__ __forceinline__ void k_mg_tail_lds_body(const TailDesc<T>& d, const T
     for (int z = zlo + tz; z <= zhi; z += bz)
       for (int y = 1 + ty; y <= q.N1 - 2; y += by)
         for (int p = tx; p < q.nxp; p += bx) f(1 + 2 * p, y, z);
+  };
+  // f(x, y, z) for each cell
+  auto cell_loop = [&](const SLev<T>& q, int ln, auto&& f) {
+    const int zlo = D == 3 ? 1 : 0, zhi = D == 3 ? q.N2 - 2 : 0;
+    const int cx = log2_up(q.N0 - 2), cl = cx + q.ly;
+    if (cl <= ln && ((zhi - zlo + 1) << cl) <= 1 << ln) {
+      const int x = 1 + (tid & ((1 << cx) - 1)), y = 1 + ((tid >> cx) & ((1 << q.ly) - 1)), z = zlo + (tid >> cl);
+      if (x <= q.N0 - 2 && y <= q.N1 - 2 && z <= zhi) f(x, y, z);
+    } else {
+      pair_loop(q, ln, [&](int x, int y, int z) {
+#pragma unroll
+        for (int o = 0; o < 2; ++o)
+          if (x + o <= q.N0 - 2) f(x + o, y, z);
+      });
+    }
   };
   // a pass's end: a barrier, or inside the first wave only the order of its LDS operations
   auto sync = [&](bool wave) {
@@ -180,22 +198,18 @@ __device__ __forceinline__ void k_mg_tail_lds_body(const TailDesc<T>& d, const T
   __syncthreads();
   for (int l = 0; l < d.n; ++l) {  // D, iD on inside (src/Poisson.jl:43-46); the first level's ϵ = r·iD
     const SLev<T> q = lev(l);
-    pair_loop(q, lnt, [&](int x, int y, int z) {
-#pragma unroll
-      for (int o = 0; o < 2; ++o) {
-        if (x + o > q.N0 - 2) continue;
-        const int I = x + o + q.s1 * y + q.s2 * z;
-        T sd = 0;
-        sd -= (q.L[I] + q.L[I + 1]);
-        sd -= (q.L[q.n + I] + q.L[q.n + I + q.s1]);
-        if (D == 3) sd -= (q.L[2 * q.n + I] + q.L[2 * q.n + I + q.s2]);
-        const T id = inv_diag(sd);
-        q.Dg[I] = sd;
-        q.iD[I] = id;
-        if (!KEEP && l == 0) {  // as restrict! left it
-          q.x[I] = 0;
-          q.e[I] = q.r[I] * id;
-        }
+    cell_loop(q, lnt, [&](int x, int y, int z) {
+      const int I = x + q.s1 * y + q.s2 * z;
+      T sd = 0;
+      sd -= (q.L[I] + q.L[I + 1]);
+      sd -= (q.L[q.n + I] + q.L[q.n + I + q.s1]);
+      if (D == 3) sd -= (q.L[2 * q.n + I] + q.L[2 * q.n + I + q.s2]);
+      const T id = inv_diag(sd);
+      q.Dg[I] = sd;
+      q.iD[I] = id;
+      if (!KEEP && l == 0) {  // as restrict! left it
+        q.x[I] = 0;
+        q.e[I] = q.r[I] * id;
       }
     });
   }
@@ -205,41 +219,33 @@ __device__ __forceinline__ void k_mg_tail_lds_body(const TailDesc<T>& d, const T
   auto jacobi = [&](int l, int ln, bool wave) {
     const SLev<T> f = lev(l);
     perbc(f, f.e, ln, wave);
-    pair_loop(f, ln, [&](int x, int y, int z) {
-#pragma unroll
-      for (int o = 0; o < 2; ++o) {
-        if (x + o > f.N0 - 2) continue;
-        const int I = x + o + f.s1 * y + f.s2 * z;
-        f.r[I] = f.r[I] - T(1) * smult(f, f.e, I);
-        f.x[I] = f.x[I] + T(1) * f.e[I];
-      }
+    cell_loop(f, ln, [&](int x, int y, int z) {
+      const int I = x + f.s1 * y + f.s2 * z;
+      f.r[I] = f.r[I] - T(1) * smult(f, f.e, I);
+      f.x[I] = f.x[I] + T(1) * f.e[I];
     });
     sync(wave);
   };
   // restrict! to level l+1, fill!(x, 0) and ϵ = r·iD there: children summed in z, y, x order
   auto restrict_to = [&](int l, int ln, bool wave) {
     const SLev<T> f = lev(l), c = lev(l + 1);
-    pair_loop(c, ln, [&](int x, int y, int z) {
+    cell_loop(c, ln, [&](int x, int y, int z) {
+      const int cc[3] = {x, y, z};
+      int a0[3], a1[3];
 #pragma unroll
-      for (int o = 0; o < 2; ++o) {
-        if (x + o > c.N0 - 2) continue;
-        const int cc[3] = {x + o, y, z};
-        int a0[3], a1[3];
-#pragma unroll
-        for (int q = 0; q < 3; ++q) {
-          const bool two = q < D && ((f.cm >> q) & 1);
-          a0[q] = two ? 2 * cc[q] - 1 : cc[q];
-          a1[q] = two ? 2 * cc[q] : cc[q];
-        }
-        T s = 0;
-        for (int kk = a0[2]; kk <= a1[2]; ++kk)
-          for (int jj = a0[1]; jj <= a1[1]; ++jj)
-            for (int ii = a0[0]; ii <= a1[0]; ++ii) s += f.r[ii + f.s1 * jj + f.s2 * kk];
-        const int Ic = x + o + c.s1 * y + c.s2 * z;
-        c.r[Ic] = s;
-        c.x[Ic] = 0;
-        c.e[Ic] = s * c.iD[Ic];
+      for (int q = 0; q < 3; ++q) {
+        const bool two = q < D && ((f.cm >> q) & 1);
+        a0[q] = two ? 2 * cc[q] - 1 : cc[q];
+        a1[q] = two ? 2 * cc[q] : cc[q];
       }
+      T s = 0;
+      for (int kk = a0[2]; kk <= a1[2]; ++kk)
+        for (int jj = a0[1]; jj <= a1[1]; ++jj)
+          for (int ii = a0[0]; ii <= a1[0]; ++ii) s += f.r[ii + f.s1 * jj + f.s2 * kk];
+      const int Ic = x + c.s1 * y + c.s2 * z;
+      c.r[Ic] = s;
+      c.x[Ic] = 0;
+      c.e[Ic] = s * c.iD[Ic];
     });
     sync(wave);
   };
@@ -324,17 +330,13 @@ __device__ __forceinline__ void k_mg_tail_lds_body(const TailDesc<T>& d, const T
     }
     if (KEEP || exact) {
       perbc(p, p.e, ln, wave);
-      pair_loop(p, ln, [&](int x, int y, int z) {
-#pragma unroll
-        for (int o = 0; o < 2; ++o) {
-          if (x + o > p.N0 - 2) continue;
-          const int I = x + o + p.s1 * y + p.s2 * z;
-          if (KEEP) {
-            p.r[I] = p.r[I] - w * smult(p, p.e, I);
-            p.x[I] = p.x[I] + w * p.e[I];
-          } else {
-            xinc(I);
-          }
+      cell_loop(p, ln, [&](int x, int y, int z) {
+        const int I = x + p.s1 * y + p.s2 * z;
+        if (KEEP) {
+          p.r[I] = p.r[I] - w * smult(p, p.e, I);
+          p.x[I] = p.x[I] + w * p.e[I];
+        } else {
+          xinc(I);
         }
       });
       sync(wave);
@@ -344,33 +346,29 @@ __device__ __forceinline__ void k_mg_tail_lds_body(const TailDesc<T>& d, const T
   auto prolong = [&](int l, int ln, bool wave) {
     const SLev<T> f = lev(l), p = lev(l + 1);
     const int N[3] = {f.N0, f.N1, f.N2};
-    pair_loop(f, ln, [&](int x, int y, int z) {
+    cell_loop(f, ln, [&](int x, int y, int z) {
+      const int c[3] = {x, y, z};
+      int q[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
 #pragma unroll
-      for (int o = 0; o < 2; ++o) {
-        if (x + o > f.N0 - 2) continue;
-        const int c[3] = {x + o, y, z};
-        int q[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
+      for (int dd = 0; dd < D; ++dd)
 #pragma unroll
-        for (int dd = 0; dd < D; ++dd)
-#pragma unroll
-          for (int k = 0; k < 3; ++k) q[dd][k] = pro_map(c[dd] + k - 1, N[dd], (d.perdir >> dd) & 1, (f.cm >> dd) & 1);
-        auto xcv = [&](int a, int b, int zz) -> T {
-          const bool ok = a >= 0 && b >= 0 && zz >= 0;
-          const T v = p.x[ok ? a + p.s1 * b + p.s2 * zz : 0];
-          return ok ? v : T(0);
-        };
-        const int I = x + o + f.s1 * y + f.s2 * z;
-        const T e0 = xcv(q[0][1], q[1][1], q[2][1]);
-        T s = e0 * f.Dg[I];
-        s += (xcv(q[0][0], q[1][1], q[2][1]) * f.L[I] + xcv(q[0][2], q[1][1], q[2][1]) * f.L[I + 1]);
-        s += (xcv(q[0][1], q[1][0], q[2][1]) * f.L[f.n + I] + xcv(q[0][1], q[1][2], q[2][1]) * f.L[f.n + I + f.s1]);
-        if (D == 3)
-          s += (xcv(q[0][1], q[1][1], q[2][0]) * f.L[2 * f.n + I] + xcv(q[0][1], q[1][1], q[2][2]) * f.L[2 * f.n + I + f.s2]);
-        const T rn = f.r[I] - w * s;
-        f.r[I] = rn;
-        f.x[I] = f.x[I] + w * e0;
-        f.e[I] = rn * f.iD[I];
-      }
+        for (int k = 0; k < 3; ++k) q[dd][k] = pro_map(c[dd] + k - 1, N[dd], (d.perdir >> dd) & 1, (f.cm >> dd) & 1);
+      auto xcv = [&](int a, int b, int zz) -> T {
+        const bool ok = a >= 0 && b >= 0 && zz >= 0;
+        const T v = p.x[ok ? a + p.s1 * b + p.s2 * zz : 0];
+        return ok ? v : T(0);
+      };
+      const int I = x + f.s1 * y + f.s2 * z;
+      const T e0 = xcv(q[0][1], q[1][1], q[2][1]);
+      T s = e0 * f.Dg[I];
+      s += (xcv(q[0][0], q[1][1], q[2][1]) * f.L[I] + xcv(q[0][2], q[1][1], q[2][1]) * f.L[I + 1]);
+      s += (xcv(q[0][1], q[1][0], q[2][1]) * f.L[f.n + I] + xcv(q[0][1], q[1][2], q[2][1]) * f.L[f.n + I + f.s1]);
+      if (D == 3)
+        s += (xcv(q[0][1], q[1][1], q[2][0]) * f.L[2 * f.n + I] + xcv(q[0][1], q[1][1], q[2][2]) * f.L[2 * f.n + I + f.s2]);
+      const T rn = f.r[I] - w * s;
+      f.r[I] = rn;
+      f.x[I] = f.x[I] + w * e0;
+      f.e[I] = rn * f.iD[I];
     });
     sync(wave);
   };
@@ -379,7 +377,7 @@ __device__ __forceinline__ void k_mg_tail_lds_body(const TailDesc<T>& d, const T
   // cold instruction lines).  ls: the first level of the first wave's part (pairs shrink with the
   // level); a pass belongs to the level it starts from on the way down, and ends at on the way up.
   int ls = d.n;
-  while (ls > 0 && lev(ls - 1).npair <= WAVE_PAIRS) --ls;
+  while (!KEEP && ls > 0 && lev(ls - 1).npair <= WAVE_PAIRS) --ls;
   const int nd = 2 * (d.n - 1), ns = nd + 2 * d.n - 1;
   bool was_wave = false;
 #pragma unroll 1
