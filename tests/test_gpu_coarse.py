@@ -296,3 +296,20 @@ def test_standalone_multigrid_levels(wl, n, perdir, T):
     for l in range(g.nlevels):
         for name in ("x", "r"):
             assert np.array_equal(g.get(name, l), o.get(name, l)), (l, name)
+
+
+@pytest.mark.parametrize("n,levels", [((128, 40, 40), 1), ((144, 96, 80), 2), ((264, 56, 56), 2), ((96, 88, 56), 1),
+                                      ((272, 56, 48), 2), ((144, 56, 48), 1), ((256, 208, 208), 1), ((96, 64, 64), 0)],
+                         ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_lean_levels(wl, n, levels, monkeypatch):
+    """Which levels the lean passes run, by the bytes of their restriction (a fifth to a quarter of the
+    plain one's): at WL_LEAN=2 those of the tests above, without it those of at least 40 and 16 MB."""
+    print("case: lean levels", n, levels, flush=True)
+    got = []
+    for mode in ("0", None if n[0] == 256 or n == (96, 64, 64) else "2"):
+        monkeypatch.delenv("WL_LEAN", raising=False) if mode is None else monkeypatch.setenv("WL_LEAN", mode)
+        sim = wl.Simulation(n, (1, 0, 0), 8, ν=0.02, body=wl.Sphere(tuple(v / 2 for v in n), 8))
+        got.append({k[1]: k[2] for k in launches(sim.flow, lambda: wl.sim_step(sim, remeasure=False))
+                    if k[0] == "inc_restrict"})
+    assert sorted(got[0]) == sorted(got[1])
+    assert [l for l in sorted(got[0]) if 3 * got[1][l] < got[0][l]] == list(range(levels))
