@@ -313,3 +313,28 @@ def test_lean_levels(wl, n, levels, monkeypatch):
                     if k[0] == "inc_restrict"})
     assert sorted(got[0]) == sorted(got[1])
     assert [l for l in sorted(got[0]) if 3 * got[1][l] < got[0][l]] == list(range(levels))
+
+
+@pytest.mark.parametrize("n", [(72, 40), (48, 24, 32), (48, 56, 40), (40, 48, 44)], ids=lambda v: "x".join(map(str, v)))
+def test_exit_f64(wl, n):
+    """exitBC! in Float64, in one workgroup and (over 2048 exit cells) gathered, against the oracle.  The
+    exit plane's two sums over its `cnt` cells are Float64 on both sides in orders of their own: at most
+    cnt·2⁻⁵³ apart each, relative to U = 1.  A step's projections spread that over u with at most a
+    factor of the box's length, and over p with that once more over Δt."""
+    print("case: exit in Float64", n, flush=True)
+    D, R, steps = len(n), min(n) / 5, 3
+    c, U = tuple(v / 2 - 0.3 for v in n), (1,) + (0,) * (D - 1)
+    sim = wl.Simulation(n, U, 2 * R, ν=R / 50, body=wl.Sphere(c, R), T=np.float64, exitBC=True)
+    o = O.OSimulation(n, U, 2 * R, nu=R / 50, bodies=[{"kind": 1, "center": c, "radius": R}], dtype=O.WL_F64,
+                      exit_bc=True)
+    for name in ("mu0", "mu1", "V"):
+        sim.flow.set(name, o.flow.get(name))
+    sim.pois.update()
+    tol = 2 * steps * int(np.prod(n[1:])) * 2.0 ** -53 * n[0]
+    for k in range(steps):
+        wl.sim_step(sim, remeasure=False)
+        o.step(remeasure=False)
+        assert sim.pois.n == o.n, k
+        eu, ep = (float(np.abs(sim.flow.get(f) - o.flow.get(f)).max()) for f in ("u", "p"))
+        print(f"  step {k}: u {eu:.2e} of {tol:.2e}, p {ep:.2e}", flush=True)
+        assert eu <= tol and ep <= tol * n[0] / min(sim.flow.Δt)
