@@ -132,7 +132,6 @@ __device__ __forceinline__ void sto2(T* base, uint32_t b, T x, T y) {
   st2((T*)((char*)base + b), x, y);
 }
 #define WL_KEEP_OFFSET(o) asm volatile("" : "+v"(o))
-// a tile's row for this wave: y uniform
 // Slabs of zc planes go round-robin to the XCDs, each walking its slab's tiles in order: a body's rows,
 // which read their coefficients, lie in few neighbouring slabs and would keep two or three XCDs busy
 // alone if each had one contiguous range (xcd_tile_id): half sweep 84 -> 77 us, prolongation 152 -> 130
@@ -142,6 +141,7 @@ __device__ __forceinline__ int lean_tile(const ZT& t) {
   const int j = b >> 3;
   return b < (slabs & ~7) * per ? ((j / per) * 8 + (b & 7)) * per + j % per : b;
 }
+// a tile's row for this wave: y uniform
 __device__ __forceinline__ PairCell lean_cell(const ZT& t) {
   PairCell c;
   const int lid = lean_tile(t);
@@ -182,7 +182,6 @@ struct PairLD {
     return s;
   }
 };
-// R: the row's element offset in a field, o: the lane's byte offset of xa
 // A plane's form: coefficients from memory, or the constants with the z walls tested, or those of a
 // plane two away from the z walls
 enum LeanMode { LEAN_MEM = 0, LEAN_WALL = 1, LEAN_MID = 2 };

@@ -1671,7 +1671,7 @@ struct FlowBase {
   virtual void pressure_force(const wl_body* b, int nb, double t, double* F) = 0;
   virtual void metrics(const wl_body* b, int nb, const double* x0, double* out) = 0;
   // the same integrals with the block partials in a caller-given device buffer `part` of at
-  // least 12·metrics_blocks() + 12 doubles (wl_flow_metrics_noalloc)
+  // least 12·metrics_blocks() doubles (wl_flow_metrics_noalloc)
   virtual int64_t metrics_blocks() const = 0;
   virtual void metrics_into(const wl_body* b, int nb, const double* x0, double* out, double* part) = 0;
   int dev = 0;  // the device current when the handle was created (its buffers and stream are there)
@@ -1723,7 +1723,7 @@ struct FlowT : FlowBase {
   // BDIM! of the rows that need only f is done by the convection kernel (WL_FUSE_BDIM=0 disables):
   // the corrector writes those rows' u to u1, k_bdim2 the others, and u1 becomes u
   T* u1 = nullptr;
-  int* rlist = nullptr;  // the inside rows left to k_bdim2_rows, then their count
+  int* rlist = nullptr;  // the inside rows left to k_bdim2_rows
   int nlist = 0;
   bool crows_ok = false;
   int crows_epoch = -1;
@@ -1750,7 +1750,7 @@ struct FlowT : FlowBase {
       const char* e = std::getenv("WL_FUSE_BDIM");
       if (!e || std::atoi(e) != 0) {
         u1 = dalloc<T>(n * D);
-        rlist = dalloc<int>((int64_t)g.N[1] * g.N[2] + 1);
+        rlist = dalloc<int>((int64_t)g.N[1] * g.N[2]);
       }
     }
     alloc_bufs(B, 3 * nblocks(box_all(g)) + 16, sizeof(T));
@@ -2353,10 +2353,10 @@ struct FlowT : FlowBase {
   void metrics(const wl_body* b, int nb, const double* x0, double* out) override {
     DBodies bs = to_dbodies(b, nb);
     const int64_t np = metrics_blocks();
-    if (mpart_n < 12 * np + 12) {
+    if (mpart_n < 12 * np) {
       dfree(mpart);
-      mpart = dalloc<double>(12 * np + 12);
-      mpart_n = 12 * np + 12;
+      mpart = dalloc<double>(12 * np);
+      mpart_n = 12 * np;
     }
     metrics_run(bs, x0, out, mpart);
   }
@@ -3055,14 +3055,14 @@ struct wl_pois_s {
 // ---------------------------------------------------------------------------------------------
 // Scratch of wl_flow_metrics_noalloc.  The block partials of the four body integrals live in this
 // file-scope device array instead of a buffer the library allocates: 12 rows of at most
-// kNoAllocBlocks block sums (blocks of 256 inside cells) plus the 12 results, 12 MiB + 96 B per
-// device, held from the library's load until the process ends.  Every call on one device shares
-// it, so calls that overlap on one device race.  Host code never passes `scratch` itself (its
+// kNoAllocBlocks block sums (blocks of 256 inside cells), 12 MiB per device, held from the library's
+// load until the process ends.  Every call on one device shares it, so calls that overlap on one
+// device race.  Host code never passes `scratch` itself (its
 // name is a host-side stand-in there): it uses the address hipGetSymbolAddress gives for the
 // device, looked up once per device with that device current.
 // ---------------------------------------------------------------------------------------------
 constexpr int64_t kNoAllocBlocks = 131072;  // 512×256×256 inside cells
-constexpr int64_t kNoAllocDoubles = 12 * kNoAllocBlocks + 12;
+constexpr int64_t kNoAllocDoubles = 12 * kNoAllocBlocks;
 __device__ __align__(256) double scratch[kNoAllocDoubles];
 constexpr int kMaxDevices = 64;
 static std::mutex g_scratch_mu;
