@@ -344,6 +344,15 @@ struct MG {
     }
   }
 
+  // Buffers that only save time (the lean passes', k_up's second residual) are taken where the card has
+  // room for 40 fields, so that a flow that fits without them still does; small fields do not ask.
+  bool plenty() const {
+    const int64_t field = lv[0].g.n * (int64_t)sizeof(T);
+    if (field < 32 << 20) return true;
+    size_t room = 0, card = 0;
+    HIPCK(hipMemGetInfo(&room, &card));
+    return (double)room > 40.0 * (double)field;
+  }
   // Level sizes (src/MultiLevelPoisson.jl:33-41,61-77); level 0 arrays may be supplied.
   void build(int D, const int* Ng, T* L0, T* x0, T* z0, int maxlevels = 10) {
     {
@@ -419,12 +428,8 @@ struct MG {
       sg.H = (int64_t)sg.Q * g0.N[1] * g0.N[2];
       se = dalloc<T>(2 * sg.H);
       lv[0].sg = sg;
-      // the lean passes' buffers (two fields and the coarser levels') only where there is plenty of room,
-      // so that what fits without them still does
-      size_t room = 0, card = 0;
-      HIPCK(hipMemGetInfo(&room, &card));
-      const bool plenty = (double)room > 40.0 * (double)(g0.n * (int64_t)sizeof(T));
-      for (int l = 0; l < (int)lv.size() && plenty && lean_level(l); ++l) {
+      const bool room = lean_level(0) && plenty();  // two fields and the coarser levels'
+      for (int l = 0; l < (int)lv.size() && room && lean_level(l); ++l) {
         Level<T>& p = lv[l];
         p.r2 = dalloc<T>(p.g.n);
         p.iD = dalloc<T>(p.g.n);
@@ -436,7 +441,8 @@ struct MG {
       }
     }
     r_home = lv[0].r;
-    if (D == 2 && up_ok(0) && perdir == 0 && !use_graphs && !smooth4_ok() && !use_gs_pair && !use_gs_dbl) fin_r = dalloc<T>(lv[0].g.n);
+    if (D == 2 && up_ok(0) && perdir == 0 && !use_graphs && !smooth4_ok() && !use_gs_pair && !use_gs_dbl && plenty())
+      fin_r = dalloc<T>(lv[0].g.n);
     if (smooth4_ok()) {
       r_alt = dalloc<T>(lv[0].g.n);
       static bool sm_attr = false;  // k_smooth4's LDS ring exceeds the default 64 KB
