@@ -338,3 +338,23 @@ def test_exit_f64(wl, n):
         eu, ep = (float(np.abs(sim.flow.get(f) - o.flow.get(f)).max()) for f in ("u", "p"))
         print(f"  step {k}: u {eu:.2e} of {tol:.2e}, p {ep:.2e}", flush=True)
         assert eu <= tol and ep <= tol * n[0] / min(sim.flow.Δt)
+
+
+@pytest.mark.parametrize("T", [np.float32, np.float64])
+@pytest.mark.parametrize("n,wide", [((64, 64, 56), 1), ((88, 88, 88), 2), ((104, 104, 96), 3)],
+                         ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else "-")
+def test_up_levels(wl, n, wide, T, monkeypatch):
+    """k_up takes a 3D level whose field has at most 400 KB: level 1 of 64x64x56 (34 680 cells) in both
+    types, of 88x88x88 (97 336) in Float32, of 104x104x96 (145 800) in neither; the same u and p as with
+    none."""
+    print("case: levels of k_up", n, T.__name__, flush=True)
+    got, first = [], 1 if wide == 1 or (wide == 2 and T is np.float32) else 2
+    for cells in (None, "0"):
+        monkeypatch.delenv("WL_UP_CELLS", raising=False) if cells is None else monkeypatch.setenv("WL_UP_CELLS", cells)
+        sim = wl.Simulation(n, (1, 0, 0), 12, ν=0.02, body=wl.Sphere(tuple(v / 2 for v in n), 12), T=T)
+        keys = launches(sim.flow, lambda: wl.sim_step(sim, remeasure=False))
+        assert min((k[1] for k in keys if k[0] == "up"), default=None) == (first if cells is None else None)
+        wl.sim_step(sim, remeasure=False)
+        got.append([sim.flow.get("u"), sim.flow.get("p"), list(sim.pois.n)])
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)

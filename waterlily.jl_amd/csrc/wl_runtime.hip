@@ -1146,11 +1146,17 @@ struct MG {
   // or by k_up on top of such a level; elsewhere its increment! is folded into the prolongation
   bool smoothed(int c, int Lt) const { return Lt > 0 && (c >= Lt || (up_ok(c) && smoothed(c + 1, Lt))); }
   // k_up in place of the separate launches of a level: a flow's own solver (nobody reads the level's
-  // r and ϵ afterwards), levels below up_cells cells.
+  // r and ϵ afterwards).  Every 2D level: step with the finest level's separate passes -> k_up, us, FP32
+  // 64x64 146 -> 122, 1024x512 274 -> 239, 4096x2048 1478 -> 1275, 8192x4096 6033 -> 4697, FP64 159 ->
+  // 135, 329 -> 292, 2410 -> 2042, 9423 -> 7422 (its tiles compute 1.72 cells for each, beside one pass
+  // over memory for five).  3D levels of at most 400 KB a field, where the launches saved are more than
+  // the tiles' 4 cells of halo on every side cost: level 1 separate -> k_up in a step, FP32 of 34 680
+  // cells 275 -> 264, 97 336 371 -> 363, 115 000 415 -> 406, 145 800 445 -> 448, 252 648 562 -> 584; FP64
+  // 34 680 365 -> 352, 66 424 447 -> 457, 97 336 509 -> 516, 145 800 658 -> 685.
   bool up_ok(int l) const {
     const Geo& g = lv[l].g;
     for (int d = 0; d < g.D; ++d) if (g.N[d] < 4) return false;
-    return fold_coarse_inc && g.n <= (up_cells >= 0 ? up_cells : (g.D == 3 ? 100000 : (int64_t)1 << 40));
+    return fold_coarse_inc && (up_cells >= 0 ? g.n <= up_cells : g.D == 2 || g.n * (int64_t)sizeof(T) <= 400000);
   }
   int64_t up_cells = -1;  // WL_UP_CELLS when the solver was built (-1: unset)
   bool fin_ok() const { return lv[0].g.D == 2 && up_ok(0) && fin_r != nullptr && perdir == 0; }
