@@ -60,10 +60,10 @@ inline LeanL<T> lean_l(const T* L, const T* iD, const uint8_t* fast, int nseg, c
   return a;
 }
 // Flags.  Pass 1, one wave per row and segment: bit i: component i has its constant (0 on wall faces)
-// over the segment's cells and those beside them, the x faces one further.
+// over the segment's cells and those beside them, the x faces one further; and 1/D of its cells (k_diag's)
 template <class T>
 __global__ void __launch_bounds__(256) k_seg_bits(Geo g, const T* __restrict__ L, T c0, T c1, T c2, int nseg,
-                                                  uint8_t* __restrict__ bits) {
+                                                  uint8_t* __restrict__ bits, T* __restrict__ iD) {
   const int64_t w = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (w >= (int64_t)g.N[1] * g.N[2] * nseg) return;  // uniform over the wavefront
@@ -73,19 +73,33 @@ __global__ void __launch_bounds__(256) k_seg_bits(Geo g, const T* __restrict__ L
   const int x0 = 2 * SEG_PAIRS * seg, x1 = min(x0 + 2 * SEG_PAIRS + 1, g.N[0] - 1);  // the cells beside included
   const int64_t base = at(g, 0, y, z);
   const T e1 = (y == 1 || y == g.N[1] - 1) ? T(0) : c1, e2 = (z == 1 || z == g.N[2] - 1) ? T(0) : c2;
+  const bool inside = y >= 1 && y <= g.N[1] - 2 && z >= 1 && z <= g.N[2] - 2;
+  const int64_t dy = inside ? g.s[1] : 0, dz = inside ? g.s[2] : 0;
+  const T *L0 = L + base, *L1 = L0 + g.n, *L2 = L1 + g.n;
   bool a0 = true, a1 = true, a2 = true;
-  for (int x = x0 + lane; x <= min(x1 + 1, g.N[0] - 1); x += 64) {
-    if (x >= 1) a0 &= same_bits(L[base + x], (x == 1 || x == g.N[0] - 1) ? T(0) : c0);
-    if (x >= 1 && x <= min(x1, g.N[0] - 2)) {
-      a1 &= same_bits(L[base + x + g.n], e1);
-      a2 &= same_bits(L[base + x + 2 * g.n], e2);
-    }
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {  // no branch before the loads: a cell beyond repeats the last one
+    const int x = x0 + lane + 64 * k;
+    const int xf = min(max(x, 1), min(x1 + 1, g.N[0] - 1)), xc = min(max(x, 1), min(x1, g.N[0] - 2));
+    const T f = L0[xf], xl = L0[xc], xh = L0[xc + 1];
+    const T yl = L1[xc], yh = L1[xc + dy], zl = L2[xc], zh = L2[xc + dz];
+    a0 &= same_bits(f, (xf == 1 || xf == g.N[0] - 1) ? T(0) : c0);
+    a1 &= same_bits(yl, e1);
+    a2 &= same_bits(zl, e2);
+    T s = 0;  // diag_at's order
+    s -= (xl + xh);
+    s -= (yl + yh);
+    s -= (zl + zh);
+    if (inside && x > x0 && x < x1) iD[base + x] = inv_diag(s);
   }
   const bool b0 = __all(a0), b1 = __all(a1), b2 = __all(a2);
   if (lane == 0) bits[w] = (uint8_t)(b0 | (b1 << 1) | (b2 << 2));
 }
 // Pass 2: every face of the segment's cells (an inside row).  Pass 3: that of the row and of its four
-// neighbours (ghost rows hold 0 and need no coefficient).
+// neighbours (ghost rows hold 0 and need no coefficient), and the level's row flags (LRows: a row whose
+// y and z faces are no walls).
+// Pass 1 is bound by its read of L: 159 us at 512x256x256, for 143 + 139 + 198 of a pass without 1/D,
+// k_diag and k_level_tables; a measure! and update! there 1325 -> 998 us.
 __global__ void __launch_bounds__(256) k_seg_uniform(Geo g, int nseg, const uint8_t* __restrict__ bits,
                                                      uint8_t* __restrict__ uni) {
   const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -97,7 +111,7 @@ __global__ void __launch_bounds__(256) k_seg_uniform(Geo g, int nseg, const uint
   uni[k] = f ? 1 : 0;
 }
 __global__ void __launch_bounds__(256) k_seg_fast(Geo g, int nseg, const uint8_t* __restrict__ uni,
-                                                  uint8_t* __restrict__ fast) {
+                                                  uint8_t* __restrict__ fast, uint8_t* __restrict__ rows) {
   const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= (int64_t)g.N[1] * g.N[2] * nseg) return;
   const int64_t row = k / nseg, sy = nseg, sz = (int64_t)g.N[1] * nseg;
@@ -107,6 +121,11 @@ __global__ void __launch_bounds__(256) k_seg_fast(Geo g, int nseg, const uint8_t
     f = uni[k] && (y == 1 || uni[k - sy]) && (y == g.N[1] - 2 || uni[k + sy]) && (z == 1 || uni[k - sz]) &&
         (z == g.N[2] - 2 || uni[k + sz]);
   fast[k] = f ? 1 : 0;
+  if (k == row * nseg) {
+    bool r = y >= 2 && y <= g.N[1] - 3 && z >= 2 && z <= g.N[2] - 3;
+    for (int s = 0; s < nseg; ++s) r = r && uni[k + s];
+    rows[row] = r ? 1 : 0;
+  }
 }
 // the flags of row y and a segment over planes zlo + lane (lanes below nz)
 template <class T>

@@ -519,7 +519,11 @@ struct MG {
       if (l == 0) ++lrow_epoch0;
       const bool img = image && l >= Lt;
       p.lrow_ok = false;
-      if (p.iD) build_lean_tables(l);
+      if (p.iD) {  // (a lean level is none of the tail's: no image)
+        build_lean_tables(l);
+        p.lrow_ok = use_lrows;
+        continue;
+      }
       if (!use_lrows && !img) continue;
       if (d.n == TAB_MAX) flush();
       TabLv<T>& q = d.lv[d.n++];
@@ -537,21 +541,23 @@ struct MG {
   }
   void build_lean_tables(int l) {
     Level<T>& p = lv[l];
-    Box b = box_inside(p.g);
-    hipLaunchKernelGGL(k_diag<T>, grid_of(b), kBlock, 0, st, p.g, b, (const T*)p.L, p.iD, 1);
-    KCK();
     p.lean_ok = true;
-    if (!use_lrows) return;
+    if (!use_lrows) {
+      Box b = box_inside(p.g);
+      hipLaunchKernelGGL(k_diag<T>, grid_of(b), kBlock, 0, st, p.g, b, (const T*)p.L, p.iD, 1);
+      KCK();
+      return;
+    }
     const int ns = lean_nseg(p.g);
     const int64_t nk = (int64_t)p.g.N[1] * p.g.N[2] * ns;
     hipLaunchKernelGGL(k_seg_bits<T>, dim3((unsigned)((nk + 3) / 4)), dim3(256), 0, st, p.g, (const T*)p.L, p.lc[0],
-                       p.lc[1], p.lc[2], ns, p.lseg);
+                       p.lc[1], p.lc[2], ns, p.lseg, p.iD);
     KCK();
     hipLaunchKernelGGL(k_seg_uniform, dim3((unsigned)((nk + 255) / 256)), dim3(256), 0, st, p.g, ns,
                        (const uint8_t*)p.lseg, p.lseg + nk);
     KCK();
     hipLaunchKernelGGL(k_seg_fast, dim3((unsigned)((nk + 255) / 256)), dim3(256), 0, st, p.g, ns,
-                       (const uint8_t*)p.lseg + nk, p.lseg + 2 * nk);
+                       (const uint8_t*)p.lseg + nk, p.lseg + 2 * nk, p.lrow);
     KCK();
   }
   bool tables_ok(const Level<T>& p) const { return (p.lrow_ok || !use_lrows) && (p.lean_ok || !p.iD); }
@@ -588,10 +594,10 @@ struct MG {
   // The lean passes (k_lean_*): levels of the colour-split solver that are coarsened in every
   // direction and too large for k_up, from the size on where a level's fields no longer stay in the
   // 256 MB last-level cache (below, the plain passes' extra values cost little and an update's 1/D and
-  // flags more).  Step with a static body, plain -> lean, us: FP32 256x128x128 880 -> 851, 320x160x160
-  // 1684 -> 1645, 384x192x192 3133 -> 2880, 512x256x256 7592 -> 6352; FP64 320x160x160 (as many bytes
-  // as FP32 402x201x201) 3442 -> 3081; with a body measured in each step 1314 -> 1329, 2425 -> 2470,
-  // 3614 -> 3521, 8121 -> 7414; 4411 -> 4124.  Coarser levels, under a lean one: at 17 MB 6352 -> 6258,
+  // flags more).  Step with a static body, plain -> lean, us: FP32 256x128x128 993 -> 983, 320x160x160
+  // 1826 -> 1854, 384x192x192 2775 -> 2564, 512x256x256 6524 -> 5404; FP64 256x128x128 1744 -> 1778,
+  // 320x160x160 3693 -> 3359; with a body measured in each step 1258 -> 1279, 2208 -> 2267, 3310 -> 3116,
+  // 7634 -> 6401; 2037 -> 2117, 4152 -> 3813.  Coarser levels, under a lean one: at 17 MB 6352 -> 6258,
   // at 14 MB 5398 -> 5471.
   bool lean_on = false;  // this projection runs them on every level that has r2
   bool lean_level(int l) const {
