@@ -304,7 +304,8 @@ def summarize(stats_csv, fetch_csv, write_csv, out_md, out_json, cmd, calib_byte
                 i = int(np.argmax(gaps))
                 lo, hi = d0[:i + 1], d0[i + 1:]
                 if np.mean(hi) > 3 * np.mean(lo):
-                    note = f" (split from {len(lo)} same-grid dispatches of a coarser level, avg {np.mean(lo):.2f} us)"
+                    note = f" (split from {len(lo)}" \
+                           f" same-grid dispatches of a coarser level or ended by their gate, avg {np.mean(lo):.2f} us)"
                     d0 = hi
             lvl0 = gmax == kmax[k] and (klead[k][0] == kn or 3 * np.mean(d0) >= klead[k][1])
             label = f"{k}@L0" if lvl0 else f"{k} (coarser levels only)"
