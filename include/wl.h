@@ -178,7 +178,8 @@ int wl_flow_cfl(wl_flow_t h, double* dt);
  * scheme, use the plain solver, and have no periodic directions, no exitBC and no warm-start
  * network attached (checked when the batch is created).  One wl_batch_step is one mom_step! of
  * every member (dt, t0, t1, dt_next: one entry per member; n_iter: two per member) with the same
- * results as wl_mom_step on each. */
+ * results as wl_mom_step on each, up to the last bits of Σr² (summed over other tiles), on which ω
+ * and the stop test hang in a solve that stagnates. */
 typedef struct wl_batch_s* wl_batch_t;
 int wl_batch_create(wl_batch_t* out, const wl_flow_t* flows, int nflows);
 int wl_batch_destroy(wl_batch_t b);

@@ -589,8 +589,10 @@ class Batch:
     """Many Simulations of different sizes stepped together: one kernel launch per stage of the
     time step for all members.  Members keep their own Δt, pois.n and fields; `step()` is one
     sim_step!(sim; remeasure=false) (src/WaterLily.jl:127-140) of every member, with the same
-    results as stepping each alone.  Members share D, T and λ, use the plain solver, and have no
-    periodic directions and no exitBC."""
+    results as stepping each alone up to the last bits of Σr²: its sums (residuals()) run over other
+    tiles there, and a solve that stagnates, whose ω or stop test hangs on them, can take another
+    ω.  Members share D, T and λ, use the plain solver, and have no periodic directions and no
+    exitBC."""
 
     def __init__(self, sims):
         self.sims = list(sims)

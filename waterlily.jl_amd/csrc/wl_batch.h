@@ -4,8 +4,9 @@
 // as the simulation's own launch maps its blocks (the XCD renumbering included), so the block
 // partial sums land in the same slots and reduce in the same order.  The per-cell work
 // is the same device body the single-simulation kernels run, so a simulation stepped in a batch
-// gives the same bits as stepped alone.  `act`, where given, skips simulations whose pressure
-// solve has converged (their blocks return at once).
+// gives the same bits as stepped alone, Σr² excepted where the single flow's finest level runs k_up or
+// the lean passes (other tiles; it decides the stop and ω alone).  `act`, where given, skips
+// simulations whose pressure solve has converged (their blocks return at once).
 #pragma once
 #include "wl_kernels.h"
 

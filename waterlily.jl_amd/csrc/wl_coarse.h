@@ -755,7 +755,7 @@ __global__ void __launch_bounds__(TAIL_FAST_PAIRS) k_mg_tail_fast(TailFast<T> d,
 // x pairs of the region (one in 2D, two in 3D), one cell of which each half sweep updates, and
 // keeps their residuals, 1/D and coefficients in registers; the LDS carries ϵ, and before it the
 // prolonged coarse values.  Every value is formed by the operations of the separate passes in their
-// order, so the results are the same bits.
+// order, so the results are the same bits; only FIN's Σr² is summed over other tiles.
 //
 // FIN (the finest level): also r −= ω·Aϵ into rout (the neighbouring blocks still read r), the next
 // Jacobi!'s ϵ = r·iD into ej and the block's Σr² into partial.

@@ -846,8 +846,8 @@ __global__ void __launch_bounds__(256) k_bc_fn(Geo g, T* __restrict__ a, const T
 // The plane's cells lie a row apart, each load a cache line of its own, and one workgroup gets about
 // 0.3 lines per ns: planes of more than EXIT_ONE cells are first gathered by a launch over the chip
 // (k_exit_gather) into u at x = 1 (q[0..cnt)), u0 at x = N0-1 (cnt..) and N0-2 (2cnt..), and the new
-// values scattered by another.  208x112x80: 48 us in one workgroup, 14 in the three launches; 142
-// cells 8 us in one.  Both ways add in the same order.
+// values scattered by another.  208x112x80: 48 us in one workgroup, 17 in the three launches; 144
+// cells in Float64 5 us in one.  Both ways add in the same order.
 constexpr int EXIT_ONE = 2048;
 __device__ __forceinline__ int64_t exit_cell(const Geo& g, int64_t t, int x) {
   const unsigned ny = g.N[1] - 2, k = (unsigned)t;

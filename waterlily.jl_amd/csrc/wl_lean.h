@@ -12,7 +12,8 @@
 //   k_lean_gs × 3      one colour of ϵ read and written each, r₂'s lines               6
 //   k_lean_increment   reads r₀, r₂, ϵ, x and the coarse x; writes x and r           6.25
 // 17.1 values.  x of a coarser level is written by the prolongation (ϵ_J + ω·e_c), of the finest by
-// the increment alone.  Each value is formed by the plain passes' operations in their order.
+// the increment alone.  Each value is formed by the plain passes' operations in their order; only Σr² is
+// summed over other tiles.
 //
 // Bound by memory: FP32 512x256x256 with a sphere, us per launch, plain -> lean: restriction 227 -> 75,
 // prolongation 190 -> 131, half sweep 81 -> 76, increment 208 -> 210 (it has taken over x's part of the

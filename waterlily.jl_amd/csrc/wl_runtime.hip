@@ -2404,9 +2404,10 @@ struct FlowT : FlowBase {
 // ---------------------------------------------------------------------------------------------
 // Batches: many uneven simulations stepped together, one launch per stage for all of them
 // (kb_* kernels, wl_batch.h).  Each member is an ordinary flow handle; the batch reads its fields
-// and multigrid levels in place, so a member gives the same bits as stepped alone.  Members share
-// D and dtype, use the plain solver, have no periodic directions and no exitBC, and have a coarse
-// tail that fits the LDS.
+// and multigrid levels in place, and every cell's value is formed by the single flow's operations, so
+// a member gives the same bits as stepped alone as long as Σr² compares alike: a 2D flow (k_up) and
+// one with lean passes sum it over tiles of their own.  Members share D and dtype, use the plain
+// solver, have no periodic directions and no exitBC, and have a coarse tail that fits the LDS.
 // ---------------------------------------------------------------------------------------------
 static int xcd_tile_host(int bid, int nb) {  // the host copy of xcd_tile_id()
   const int q = nb >> 3, rr = nb & 7, x = bid & 7, k = bid >> 3;
